@@ -72,8 +72,12 @@ __global__ __launch_bounds__(64 * PREP_WAVES) void attn_prep_kernel(
     const int kh = kind == 0 ? r : (kind == 1 ? r - nh : r - nh - nkv);
     const float* src = kind == 0 ? q + (size_t)t * qts + (size_t)kh * 2 * HDK
                                  : (kind == 1 ? k : v) + (size_t)t * kts + (size_t)kh * HDK;
-    V x = {};
+    // The head's norm weights go out with it: loaded where they are used, after the table's barrier
+    // and the sum of squares, they cost a second memory round trip on the path of a one-token call.
+    const float* wt = kind == 0 ? qw : kw;
+    V x = {}, wv = {};
     if (live) x = *(const V*)(src + E * l);
+    if (live && kind != 2 && wt) wv = *(const V*)(wt + E * l);
     for (int i = threadIdx.x; i < half; i += 64 * PREP_WAVES) {
         float c = 1.0f, s = 0.0f;
         if (!rope_use_e(i, s0, s1, s2, s3)) rope_angle(p, i, tsc, c, s);
@@ -88,9 +92,6 @@ __global__ __launch_bounds__(64 * PREP_WAVES) void attn_prep_kernel(
         for (int j = 0; j < E; ++j) ss += x[j] * x[j];
         ss = wave_sum(ss);
         const float sc = 1.0f / sqrtf(ss / (float)HDK + eps);
-        const float* wt = kind == 0 ? qw : kw;
-        V wv;
-        if (wt) wv = *(const V*)(wt + E * l);
 #pragma unroll
         for (int j = 0; j < E; ++j) x[j] = wt ? (x[j] * sc) * wv[j] : x[j] * sc;
         // Rotation of the pair (e, e + half) for e < half: both partners sit in lanes half/E apart
