@@ -154,27 +154,30 @@ __global__ __launch_bounds__(256) void gdn_conv_l2_kernel(const float* __restric
 // The same pass with 16-byte accesses (strides and bases 16-byte aligned, cd % 256 == 0): lane l
 // holds channels 256*wb + 4l .. 4l+3 of wave block wb, so lanes 0-31 and 32-63 each hold one
 // 128-channel head and a head's sum of squares is a reduction over its 32 lanes (DPP within the
-// 16-lane rows, then a row swap). A quarter of the memory instructions of the scalar form.
-template <int K, typename OutT>
+// 16-lane rows, then a row swap). A quarter of the memory instructions of the scalar form. For prompts
+// of several runs of TMAX tokens: the new state (and a checkpoint) is not written here, since other
+// runs still read the old one.
+template <int K, typename OutT, int TMAX>
 __global__ __launch_bounds__(256) void gdn_conv_l2_v4_kernel(const float* __restrict__ x, int xts,
-                                                             const float* __restrict__ w, float* __restrict__ state,
-                                                             OutT* __restrict__ out, int ots, int cd, int nt, int TT,
-                                                             int nnorm, float eps, float* __restrict__ ck,
-                                                             int ck_after) {
-    constexpr int TMAX = 16;   // tokens per run (the host passes TT <= TMAX)
+                                                             const float* __restrict__ w,
+                                                             const float* __restrict__ state, OutT* __restrict__ out,
+                                                             int ots, int cd, int nt, int nnorm, float eps) {
     const int wb = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
     if (wb >= cd / 256) return;   // whole waves
     const int ch = 256 * wb + 4 * l;
     const bool norm = (ch >> 7) < nnorm;   // uniform over each 32-lane half
-    const int t0 = blockIdx.y * TT, n = min(nt, t0 + TT) - t0;
+    const int t0 = blockIdx.y * TMAX, n = min(nt, t0 + TMAX) - t0;
     f4 xs[TMAX], wt[K], win[K - 1];
 #pragma unroll
     for (int j = 0; j < TMAX; ++j) xs[j] = ld_f4(x + (size_t)(t0 + min(j, n - 1)) * xts + ch);
+    // taps of channel ch + e: floats (ch + e) * K .. + K, the lane's 4K floats as K aligned f4
+    f4 wv[K];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {   // taps of channel ch + e are w[(ch + e) * K .. + K)
+    for (int i = 0; i < K; ++i) wv[i] = ld_f4(w + (size_t)ch * K + 4 * i);
 #pragma unroll
-        for (int i = 0; i < K; ++i) wt[i][e] = w[(size_t)(ch + e) * K + i];
-    }
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < K; ++i) wt[i][e] = wv[(e * K + i) >> 2][(e * K + i) & 3];
 #pragma unroll
     for (int i = 0; i < K - 1; ++i) {
         const int tt = t0 - (K - 1) + i;
@@ -203,14 +206,6 @@ __global__ __launch_bounds__(256) void gdn_conv_l2_v4_kernel(const float* __rest
 #pragma unroll
         for (int i = 0; i + 1 < K - 1; ++i) win[i] = win[i + 1];
         win[K - 2] = xs[j];
-        if (ck && t0 + j == ck_after && gridDim.y == 1) {
-#pragma unroll
-            for (int i = 0; i < K - 1; ++i) *(f4*)(ck + (size_t)i * cd + ch) = win[i];
-        }
-    }
-    if (gridDim.y == 1) {
-#pragma unroll
-        for (int i = 0; i < K - 1; ++i) *(f4*)(state + (size_t)i * cd + ch) = win[i];
     }
 }
 
@@ -711,41 +706,51 @@ hipError_t launch_gdn_conv(const float* x, int xts, const float* w, float* state
 
 template <typename OutT>
 hipError_t launch_gdn_conv_l2(const float* x, int xts, const float* w, float* state, OutT* out, int ots, int cd,
-                              int nt, int K, int nnorm, float eps, float* ck, int ck_after, hipStream_t st) {
+                              int nt, int K, int nnorm, float eps, float* ck, int ck_after, hipStream_t st,
+                              bool defer_state) {
     const int TT = nt <= 16 ? nt : 16;
     const dim3 grid((cd / 128 + 3) / 4, (nt + TT - 1) / TT);
     // 16-byte form for prompts (several 16-token runs) when every access is 16-byte aligned and a
     // wave's 256 channels are whole; a decode or verify token keeps twice the waves of the scalar form
-    const bool v4 = nt > 16 && cd % 256 == 0 && xts % 4 == 0 && ots % 4 == 0 && ((uintptr_t)x & 15) == 0 &&
-                    ((uintptr_t)out & 15) == 0 && ((uintptr_t)state & 15) == 0 && (!ck || ((uintptr_t)ck & 15) == 0);
-    const dim3 grid4((cd / 256 + 3) / 4, (nt + TT - 1) / TT);
+    // (a grid has at most 65535 rows of runs: longer prompts take the scalar form's 16-token runs)
+    const bool v4 = nt > 16 && nt <= 8 * 65535 && cd % 256 == 0 && xts % 4 == 0 && ots % 4 == 0 && ((uintptr_t)x & 15) == 0 &&
+                    ((uintptr_t)out & 15) == 0 && ((uintptr_t)state & 15) == 0 && ((uintptr_t)w & 15) == 0 && (!ck || ((uintptr_t)ck & 15) == 0);
+    // Tokens a run: 4 for prompts of up to 2^23 values (x + its f16 or f32 output stay near the L2s and the
+    // pass is bound by one round trip per wave with too few waves in flight), 8 beyond (each run reads
+    // the K-1 rows before it again, which then come from memory). Prefill layer, 16 / 8 / 4 tokens a run:
+    // 24 tokens x 8192 channels 19.3 / 16.9 / 15.9 us, 500 34.5 / 32.9 / 32.0, 1000 48.7 / 46.3 / 45.3;
+    // 500 x 10240 47.0 / 44.7 / 44.0, 1000 72.8 / 68.9 / 71.1, 4096 248 / 245 / 257 us.
+    const int TT4 = (size_t)nt * cd <= (1u << 23) ? 4 : 8;
+    const dim3 grid4((cd / 256 + 3) / 4, (nt + TT4 - 1) / TT4);
+#define IT_L2_V4(KK, TM)                                                                                            \
+    gdn_conv_l2_v4_kernel<KK, OutT, TM><<<grid4, 256, 0, st>>>(x, xts, w, state, out, ots, cd, nt, nnorm, eps)
 #define IT_L2_RUN(KK, TM)                                                                                           \
     gdn_conv_l2_kernel<KK, OutT, TM><<<grid, 256, 0, st>>>(x, xts, w, state, out, ots, cd, nt, TT, nnorm, eps, ck,     \
                                                            ck_after)
 #define IT_CONVL2(KK)                                                                                               \
     if (ck && grid.y > 1)                                                                                           \
         gdn_conv_state_kernel<KK><<<(cd + 255) / 256, 256, 0, st>>>(x, xts, state, ck, cd, ck_after + 1);          \
-    if (v4)                                                                                                         \
-        gdn_conv_l2_v4_kernel<KK, OutT><<<grid4, 256, 0, st>>>(x, xts, w, state, out, ots, cd, nt, TT, nnorm, eps,  \
-                                                               ck, ck_after);                                       \
+    if (v4 && TT4 == 4) IT_L2_V4(KK, 4);                                                                            \
+    else if (v4) IT_L2_V4(KK, 8);                                                                                   \
     else if (TT <= 1) IT_L2_RUN(KK, 1);                                                                             \
     else if (TT <= 2) IT_L2_RUN(KK, 2);                                                                             \
     else if (TT <= 4) IT_L2_RUN(KK, 4);                                                                             \
     else IT_L2_RUN(KK, 16);                                                                                         \
-    if (grid.y > 1) gdn_conv_state_kernel<KK><<<(cd + 255) / 256, 256, 0, st>>>(x, xts, state, state, cd, nt);
+    if (grid.y > 1 && !defer_state) gdn_conv_state_kernel<KK><<<(cd + 255) / 256, 256, 0, st>>>(x, xts, state, state, cd, nt);
     switch (K) {
         case 2: IT_CONVL2(2) break;
         case 3: IT_CONVL2(3) break;
         default: IT_CONVL2(4) break;
     }
 #undef IT_CONVL2
+#undef IT_L2_V4
 #undef IT_L2_RUN
     return hipGetLastError();
 }
 template hipError_t launch_gdn_conv_l2<float>(const float*, int, const float*, float*, float*, int, int, int, int,
-                                                int, float, float*, int, hipStream_t);
+                                                int, float, float*, int, hipStream_t, bool);
 template hipError_t launch_gdn_conv_l2<_Float16>(const float*, int, const float*, float*, _Float16*, int, int, int,
-                                                   int, int, float, float*, int, hipStream_t);
+                                                   int, int, float, float*, int, hipStream_t, bool);
 
 hipError_t launch_l2norm(float* x, int ts, int nheads, int d, int nt, float eps, hipStream_t st) {
     const int rows = nheads * nt;

@@ -65,10 +65,12 @@ hipError_t launch_attn_flash_split(const float* q, int qts, const uint16_t* kc, 
 // ck / ck_after: optional checkpoint of the state after token ck_after (null = none).
 hipError_t launch_gdn_conv(const float* x, int xts, const float* w, float* state, float* out, int ots, int cd, int nt,
                            int K, float* ck, int ck_after, hipStream_t st);
-// OutT float or _Float16 (the conv output as f16 for the one-call GDN prefill)
+// OutT float or _Float16 (the conv output as f16 for the one-call GDN prefill). defer_state: with more
+// than 16 tokens the new conv state is left to the caller (ConvTail).
 template <typename OutT>
 hipError_t launch_gdn_conv_l2(const float* x, int xts, const float* w, float* state, OutT* out, int ots, int cd,
-                              int nt, int K, int nnorm, float eps, float* ck, int ck_after, hipStream_t st);
+                              int nt, int K, int nnorm, float eps, float* ck, int ck_after, hipStream_t st,
+                              bool defer_state = false);
 hipError_t launch_l2norm(float* x, int ts, int nheads, int d, int nt, float eps, hipStream_t st);
 hipError_t launch_gdn_decode_fused(const float* x, int xts, const float* cw, int K, const float* cst_in, float* cst_out,
                                    const float* br, const float* ar, int bts, const float* dt, const float* a,
@@ -84,11 +86,19 @@ hipError_t launch_gdn_step_head(const float* co, int cts, const float* br, const
 hipError_t launch_gdn_gated_norm(const float* o, int ots, const float* z, int zts, const float* w, float eps,
                                  float* out, int outs, int nv, int nt, hipStream_t st);
 size_t gdn_chunked_scratch_bytes(int nt, int nv, int S, bool f16_conv);
+// The conv state after a prompt of more than 16 tokens, the last K-1 rows of the layer input x, written
+// by workgroups that launch_gdn_chunked adds to its first kernel (state == null: nothing to write).
+struct ConvTail {
+    const float* x = nullptr;
+    int xts = 0;
+    float* state = nullptr;
+    int cd = 0, K = 0;
+};
 // CoT float (it_gdn_chunked) or _Float16 (the conv output of the one-call GDN prefill)
 template <typename CoT>
 hipError_t launch_gdn_chunked(const CoT* co, int cts, const float* br, const float* ar, int bts, const float* dt,
                               const float* a, float* state, float* out, int ots, int nt, int nv, int nk, void* scratch,
-                              hipStream_t st);
+                              hipStream_t st, const ConvTail& tail = ConvTail());
 
 // f16 matrix-core rate probe: wgs workgroups of 4 waves, each wave 4 x iters 32x32x16 MFMAs;
 // out receives wgs * 256 floats.

@@ -467,3 +467,29 @@ def test_prefill_one_call_config5(dev):
     assert assert_argmax_agrees(out[-1:], out_ref[-1:]) == 0
     near = assert_argmax_agrees(out, out_ref)
     print(f"config5 one call: {near} near-tie argmax rows of {nt} over the whole prompt")
+
+
+@pytest.mark.parametrize("nt,nv,nk,K", [(17, 8, 4, 4), (18, 8, 4, 3), (19, 4, 2, 2), (24, 8, 4, 4), (67, 48, 16, 4),
+                                        (1029, 32, 16, 4)])
+def test_conv_runs_and_prefill_conv_state(dev, nt, nv, nk, K):
+    """The prompt conv at the edges of its 4-token runs, and of its 8-token runs (above 2^23 values):
+    against the oracle; and the conv state that the one-call prefill leaves is the layer input's
+    last K-1 rows. Taps off by a float take the scalar form: the same to rounding."""
+    announce(f"conv runs nt={nt} nv={nv} K={K}")
+    d = gdn_inputs(51 + nt, nt=nt, nv=nv, nk=nk)
+    w, st0 = d["w"][:, :K].copy(), d["conv_state"][:K - 1].copy()
+    want, wst = oracle.gdn_conv(d["x"], w, st0)
+    want = oracle.l2norm_heads(want, 2 * nk, 128)
+    x, wd = dev_f32(d["x"], dev), dev_f32(w, dev)
+    st = dev_f32(st0, dev)
+    got = host(ops.gdn_conv_l2norm(x, wd, st, 2 * nk))
+    np.testing.assert_allclose(got, want, rtol=1e-5, atol=1e-6)
+    np.testing.assert_array_equal(host(st), wst)
+    off = torch.empty(w.size + 1, device=dev)[1:].view(w.shape)
+    off.copy_(wd)
+    st = dev_f32(st0, dev)
+    np.testing.assert_allclose(host(ops.gdn_conv_l2norm(x, off, st, 2 * nk)), got, rtol=2e-6, atol=1e-7)
+    st = dev_f32(st0, dev)
+    ops.gdn_prefill(x, wd, st, dev_f32(d["beta_raw"], dev), dev_f32(d["alpha_raw"], dev), dev_f32(d["dt"], dev),
+                    dev_f32(d["a"], dev), dev_f32(d["state"], dev), nv, nk)
+    np.testing.assert_array_equal(host(st), wst)
