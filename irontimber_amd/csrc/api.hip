@@ -828,9 +828,12 @@ int it_gdn_prefill(const float* x, int xts, const float* w, int K, float* conv_s
     _Float16* co = (_Float16*)scratch;
     void* rec = (char*)scratch + gdn_prefill_co_bytes(nt, nv, nk, S);
     hipStream_t st = (hipStream_t)stream;
-    if (check(it::launch_gdn_conv_l2(x, xts, w, conv_state, co, cd, cd, nt, K, 2 * nk, eps, nullptr, 0, st), who))
+    if (check(it::launch_gdn_conv_l2(x, xts, w, conv_state, co, cd, cd, nt, K, 2 * nk, eps, nullptr, 0, st, true), who))
         return -1;
-    return check(it::launch_gdn_chunked(co, cd, br, ar, bts, dt, a, state, out, ots, nt, nv, nk, rec, st), who);
+    // up to 16 tokens the conv kernel has written its state itself
+    it::ConvTail tail;
+    if (nt > 16) tail = it::ConvTail{x, xts, conv_state, cd, K};
+    return check(it::launch_gdn_chunked(co, cd, br, ar, bts, dt, a, state, out, ots, nt, nv, nk, rec, st, tail), who);
 }
 
 // ---- reference-shaped policy (src/vk/mod.rs:130-220) -------------------------------------------

@@ -91,7 +91,17 @@ template <typename CoT>
 __global__ __launch_bounds__(PREP_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(CoT) == 2 ? 6 : 4)))
 void gdn_chunk_prep(const CoT* __restrict__ co, int cts, const float* __restrict__ br, const float* __restrict__ ar,
                     int bts, const float* __restrict__ dt, const float* __restrict__ A, int nt, int nv, int nk,
-                    char* __restrict__ scr) {
+                    char* __restrict__ scr, ConvTail tail) {
+    const int nch = (nt + C - 1) / C;
+    if ((int)blockIdx.x >= nch * nv) {
+        // the workgroups past the chunks write the conv state: the conv kernel, whose runs read the
+        // old one, is done. A launch of its own cost 4-5 us of a 58 us layer at 500 tokens.
+        const int ch = ((int)blockIdx.x - nch * nv) * PREP_THREADS + (int)threadIdx.x;
+        if (ch < tail.cd)
+            for (int i = 0; i < tail.K - 1; ++i)
+                tail.state[(size_t)i * tail.cd + ch] = tail.x[(size_t)(nt - (tail.K - 1) + i) * tail.xts + ch];
+        return;
+    }
     // an f16 conv output is exact in f16, so its hi/lo splits have lo == 0 and the K K^T / Q K^T
     // products need only the hi x hi term (bit-identical to the three-term form); the lo plane of
     // the K tile is then not kept, and the 48 KB of LDS leave room for three workgroups per CU
@@ -102,7 +112,6 @@ void gdn_chunk_prep(const CoT* __restrict__ co, int cts, const float* __restrict
     __shared__ float sG[C], sB[C];
     __shared__ __align__(16) float TdT[4][16][20];           // TdT[i][c][r] = (I + A'_ii)^-1 [r][c]
 
-    const int nch = (nt + C - 1) / C;
     int c, h;
     prep_wg(blockIdx.x, nch, nv, nk, c, h);
     const int t0 = c * C, L = min(C, nt - t0);
@@ -704,9 +713,11 @@ __global__ __launch_bounds__(SCAN_THREADS) void gdn_chunk_scan(const char* __res
 template <typename CoT>
 hipError_t launch_gdn_chunked(const CoT* co, int cts, const float* br, const float* ar, int bts, const float* dt,
                               const float* a, float* state, float* out, int ots, int nt, int nv, int nk, void* scratch,
-                              hipStream_t st) {
+                              hipStream_t st, const ConvTail& tail) {
     const int nch = (nt + C - 1) / C;
-    gdn_chunk_prep<<<dim3(nch * nv), PREP_THREADS, 0, st>>>(co, cts, br, ar, bts, dt, a, nt, nv, nk, (char*)scratch);
+    const int twg = tail.state ? (tail.cd + PREP_THREADS - 1) / PREP_THREADS : 0;   // conv state workgroups
+    gdn_chunk_prep<<<dim3(nch * nv + twg), PREP_THREADS, 0, st>>>(co, cts, br, ar, bts, dt, a, nt, nv, nk, (char*)scratch,
+                                                                  tail);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     // linear grid of 8 * NCB * ceil(nv / 8) workgroups, mapped to (head, column block) in-kernel
@@ -715,8 +726,10 @@ hipError_t launch_gdn_chunked(const CoT* co, int cts, const float* br, const flo
     return hipGetLastError();
 }
 template hipError_t launch_gdn_chunked<float>(const float*, int, const float*, const float*, int, const float*,
-                                              const float*, float*, float*, int, int, int, int, void*, hipStream_t);
+                                              const float*, float*, float*, int, int, int, int, void*, hipStream_t,
+                                              const ConvTail&);
 template hipError_t launch_gdn_chunked<_Float16>(const _Float16*, int, const float*, const float*, int, const float*,
-                                                 const float*, float*, float*, int, int, int, int, void*, hipStream_t);
+                                                 const float*, float*, float*, int, int, int, int, void*, hipStream_t,
+                                                 const ConvTail&);
 
 }  // namespace it
