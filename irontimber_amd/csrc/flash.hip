@@ -776,15 +776,36 @@ hipError_t launch_attn_flash(const float* q, int qts, const uint16_t* kc, const 
     return hipGetLastError();
 }
 
+// Keys per split of a launch that one pass would leave short of workgroups (fewer than 128), 0 for one
+// pass. One workgroup fits a CU, so a launch takes whole rounds of 256 workgroups, each as long as its
+// longest split: the split minimises
+//   rounds * (1.8 us a 64-key tile + 12 us a workgroup) + 1 us per 32 workgroups of records to merge
+// over the splits into 1 .. 32 ranges (what the row merge holds: 24 tokens at 8000 in 63 ranges 24.4, in 32
+// 21.2 us), counting the workgroups that have keys to see.
+// The split that reaches 256 workgroups without regard to the rounds, which this rule replaces, left a
+// second round of a few workgroups at most sizes: 441 tokens at position 7560 (280 workgroups) 110 against
+// 77 us, 24/4 heads with 64 tokens at 4096 34 against 26 us, 256 at 5000 75 against 49 us, 512 at 5000
+// 132 against 99 us; where it had met a whole round (16/2 heads, 64 and 512 tokens) the choice is the same.
 int flash_split_chunk(int pos0, int nt, int nh, int nkv) {
-    const int R = nt * (nh / nkv);
-    const int wgs = (R + BM - 1) / BM * nkv;
+    const int G = nh / nkv, R = nt * G, nrt = (R + BM - 1) / BM, wgs = nrt * nkv;
     const int keys = pos0 + nt;
     if (wgs >= 128 || keys <= 4 * BN) return 0;
-    const int want = (256 + wgs - 1) / wgs;                       // splits to reach ~256 workgroups
-    int chunk = ((keys + want - 1) / want + BN - 1) / BN * BN;    // multiple of the 64-key tile
-    chunk = chunk < 2 * BN ? 2 * BN : chunk;
-    return chunk >= keys ? 0 : chunk;
+    const int smax = wgs <= 64 ? 32 : (2 * 256 + wgs - 1) / wgs;   // (beyond: always more rounds)
+    long best_cost = -1;
+    int best = 0;
+    for (int s = 1; s <= smax; ++s) {
+        const int c = ((keys + s - 1) / s + BN - 1) / BN * BN;
+        if (c == best) continue;
+        long n = 0;
+        for (int rt = 0; rt < nrt; ++rt) n += (pos0 + (min(R, rt * BM + BM) - 1) / G + c) / c;   // ceil(keys seen / c)
+        n *= nkv;
+        const long cost = (n + 255) / 256 * (288L * (c / BN) + 1920) + (s > 1 ? 5 * n : 0);   // 1/160 us
+        if (best_cost < 0 || cost < best_cost) {
+            best_cost = cost;
+            best = c;
+        }
+    }
+    return best >= keys ? 0 : best;
 }
 
 hipError_t launch_attn_flash_split(const float* q, int qts, const uint16_t* kc, const uint16_t* vc, int kvd, int pos0,

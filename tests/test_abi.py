@@ -207,6 +207,19 @@ def test_plan_fits_reference_room_sweep(tmp_path, nh, nkv):
     assert plans == 8126464 and grown > 0
 
 
+@pytest.mark.parametrize("pos0,nt,nh,nkv", [(4096, 64, 24, 4), (8128, 64, 24, 4), (7560, 441, 16, 2),
+                                            (5000, 256, 24, 4), (5000, 512, 24, 4), (7680, 512, 16, 2),
+                                            (8000, 24, 16, 2), (1000, 16, 16, 2)])
+def test_flash_split_fills_whole_rounds(pos0, nt, nh, nkv):
+    """Key splits of prompt chunks: at most 256 workgroups (one round of one a CU), at least half of
+    them where there are keys enough, at most the 32 records a row that the row merge holds."""
+    rc, kernel, chunk, _ = plan(pos0, nt, nh, nkv, 1 << 40)
+    assert (rc, kernel) == (0, 2) and chunk % 64 == 0 and 0 < chunk < pos0 + nt
+    splits = -(-(pos0 + nt) // chunk)
+    wgs = -(-nt * (nh // nkv) // 128) * nkv * splits
+    assert wgs <= 256 and splits <= 32 and (wgs > 128 or splits >= 16)
+
+
 def plan(pos0, nt, nh, nkv, budget):
     k, c, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
     rc = _lib.lib().it_attn_plan(pos0, nt, 256, nh, nkv, budget, ctypes.byref(k), ctypes.byref(c), ctypes.byref(b))

@@ -152,6 +152,15 @@ def test_flash_whole_prompt_8192(dev):
         assert np.abs(whole - chunked).max() <= TOL
 
 
+@pytest.mark.parametrize("ctx,nt,nh,nkv", [(4160, 64, 24, 4), (8001, 441, 16, 2), (5256, 256, 24, 4),
+                                           (8024, 24, 16, 2), (317, 17, 16, 2), (700, 700, 16, 2), (3700, 700, 16, 2)])
+def test_flash_split_plans(dev, ctx, nt, nh, nkv):
+    """The automatic key splits of prompt calls over both head geometries, ragged lengths and the
+    smallest and largest row counts that are split, against the oracle."""
+    got, want = run_case(dev, 61, ctx, nt, nh, nkv)
+    assert np.isfinite(got).all() and np.abs(got - want).max() <= TOL
+
+
 @pytest.mark.parametrize("chunk", [0, 64, 192, 640])
 def test_flash_f32_records(dev, chunk):
     """The key-split flash path with lossless f32 records (kernel 3: the split-K kernels' 260-word
