@@ -41,6 +41,19 @@ def test_f32kv_matches_oracle(dev, rows, nt, nh, nkv):
     assert_argmax_agrees(got, want)
 
 
+@pytest.mark.parametrize("rows,nt,nh,nkv", [(700, 3, 16, 2), (700, 4, 16, 2), (1000, 5, 16, 2), (1500, 6, 24, 4),
+                                            (3000, 64, 24, 4), (130, 17, 2, 2), (129, 33, 16, 1)])
+def test_f32kv_two_row_blocks(dev, rows, nt, nh, nkv):
+    """Calls of two 16-row blocks a workgroup, four waves each: a block short of rows, whole blocks,
+    30 rows of 6 heads, the second block's rows in the first group only, 16 heads over one KV head;
+    one and several tiles a split. The bound is that of the calls above."""
+    announce(f"f32kv two blocks rows={rows} nt={nt} nh={nh} nkv={nkv}")
+    q, k, v = f32kv_inputs(rows + nt, rows, nt, nh, nkv)
+    got = host(ops.attn_f32kv(dev_f32(q, dev), dev_f32(k, dev), dev_f32(v, dev), rows - nt, nh, nkv))
+    want = oracle.attn_f32kv(q, k, v, rows - nt, nh, nkv)
+    assert np.isfinite(got).all() and np.abs(got - want).max() <= 2e-5
+
+
 @pytest.mark.parametrize("nh,nkv,hd", GEOMS)
 @pytest.mark.parametrize("pos0,nt", CASES)
 def test_f32kv_r012_known_answer(dev, pos0, nt, nh, nkv, hd):
