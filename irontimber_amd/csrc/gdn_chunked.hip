@@ -15,8 +15,8 @@
 // products, ~f32 accurate); Kh and P^T solve (I + A')^T [Z1 | Z2] = [diag(e^{G_last-G}) K | (D *
 // Q K^T)^T] by blocked backward substitution (16x16 diagonal inverses, MFMA hi+lo products), then
 // scale rows by beta. From an f32 conv output it also writes the chunk's q and k rows as f16.
-// Kernel 2 (gdn_chunk_scan, one workgroup per (16-column block of the state, V head)) walks the
-// chunks in order with its 128x16 slice of S in MFMA accumulators; S0 and Y enter the products as
+// Kernel 2 (gdn_chunk_scan, one workgroup per (16- or 32-column block of the state, V head)) walks the
+// chunks in order with its slice of S in MFMA accumulators; S0 and Y enter the products as
 // f16 hi+lo pairs through LDS, so the state path keeps f32 accuracy. It reads q, k and its V
 // columns from the conv output in place (q and k from the record for an f32 conv output), so a
 // record holds 25 KiB per chunk and V head (57 KiB with the f16 q and k rows).
@@ -371,22 +371,18 @@ void gdn_chunk_prep(const CoT* __restrict__ co, int cts, const float* __restrict
 }
 
 // ------------------------------------------------------------------------------------------------
-constexpr int CW = 16;         // state columns per scan workgroup
-constexpr int NCB = SD / CW;   // column blocks of the state per head
-constexpr int NI = CW / 16;    // 16-column MFMA tiles per workgroup
-
 // Workgroup barrier for LDS data written by the waves themselves (ds_write): waits for this wave's
 // LDS operations only, not for the next chunk's operand loads, which are in flight by design.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-// One chunk's operands for one column block, staged in LDS by the direct global->LDS path. Rows
-// are XOR-swizzled by 16-byte chunk so the operand reads of 16 consecutive rows hit distinct
+// One chunk's operands for one block of CW state columns, staged in LDS by the direct global->LDS path.
+// Rows are XOR-swizzled by 16-byte chunk so the operand reads of 16 consecutive rows hit distinct
 // banks: 256-byte rows (k, q) by row & 15, 128-byte rows (Kh^T, P) by (row >> 1) & 7 (two rows
-// share a 256-byte bank window). V holds this block's CW columns of the conv output's V rows (f16
+// share a 256-byte bank window). V holds this block's columns of the conv output's V rows (f16
 // or f32, as the conv output); T the decay table.
-template <typename CoT>
+template <typename CoT, int CW>
 struct ScanStage {
     _Float16 K[C * SD];      // [token][dim]
     _Float16 Q[C * SD];      // [token][dim]
@@ -402,11 +398,11 @@ __device__ __forceinline__ int swz128(int r) { return (r >> 1) & 7; }
 // the k and q rows (scan_stage_kq: from `qb`, row r at qb + min(r, L-1) * pitch, its k row koff
 // halves further; 4 + 4 instructions a wave), and the rest (scan_stage_rest: Kh^T, P and (part 0)
 // the decay table from the record `rec`, V rows from `vb`, row r at vb + min(r, L-1) * cts; Kh^T
-// 4, P 2, V 2 or 4 in all, +1). Instructions of 64 lanes x 16 bytes; lane l lands at byte 16*l of
+// 4, P 2, V scan_v_loads, +1). Instructions of 64 lanes x 16 bytes; lane l lands at byte 16*l of
 // its instruction's 1 KB.
-template <typename CoT>
+template <typename CoT, int CW>
 __device__ __forceinline__ void scan_stage_kq(const _Float16* __restrict__ qb, int pitch, int koff, int L,
-                                              ScanStage<CoT>& B, int part, int l) {
+                                              ScanStage<CoT, CW>& B, int part, int l) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {   // 4 rows of 256 B per instruction
         const int i = 4 * part + k, r = 4 * i + (l >> 4), j = (l & 15) ^ swz256(r);
@@ -418,9 +414,11 @@ __device__ __forceinline__ void scan_stage_kq(const _Float16* __restrict__ qb, i
 constexpr int SCAN_KQ_LOADS = 8;   // instructions of scan_stage_kq per loader wave
 constexpr int SCAN_TOUCH_AHEAD = 3;   // chunks between a chunk's L2 touch and its staging
 
-template <typename CoT>
+// V instructions in all: C rows of CW columns
+template <typename CoT, int CW> constexpr int scan_v_loads() { return C * CW * (int)sizeof(CoT) / 1024; }
+template <typename CoT, int CW>
 __device__ __forceinline__ void scan_stage_rest(const char* __restrict__ rec, const CoT* __restrict__ vb, int cts,
-                                                int L, ScanStage<CoT>& B, int part, int l) {
+                                                int L, ScanStage<CoT, CW>& B, int part, int l) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {   // Kh^T: 8 rows of 128 B per instruction
         const int i = 4 * part + k, r = 8 * i + (l >> 3), j = (l & 7) ^ swz128(r);
@@ -432,8 +430,7 @@ __device__ __forceinline__ void scan_stage_rest(const char* __restrict__ rec, co
         __builtin_amdgcn_global_load_lds(rec + OFF_P + r * C * 2 + 16 * j, (lds_void*)(B.P + 8 * i * C), 16, 0, 0);
     }
     constexpr int VL = CW * (int)sizeof(CoT) / 16;   // 16-byte lanes per V row
-    constexpr int NVI = C * VL / 64;                  // V instructions in all (2 or 4)
-    for (int i = part; i < NVI; i += 4) {             // uniform
+    for (int i = part; i < scan_v_loads<CoT, CW>(); i += 4) {   // uniform
         const int r = (64 / VL) * i + l / VL;
         __builtin_amdgcn_global_load_lds((const void*)(vb + (size_t)min(r, L - 1) * cts + 16 / sizeof(CoT) * (l % VL)),
                                          (lds_void*)(B.V + (64 / VL) * i * CW), 16, 0, 0);
@@ -443,29 +440,42 @@ __device__ __forceinline__ void scan_stage_rest(const char* __restrict__ rec, co
 
 // Scan workgroup: 8 compute waves + 4 loader waves. The dependency chain per chunk is
 // Y = V - e^G K S0 and S1 = e^{G_last} S0 + Kh^T Y; the output O = e^G Q S0 + P Y hangs off it.
-// Waves 0-3 ("chain") run the chain for chunk c while waves 4-7 ("output") compute O of chunk c-1
-// from the previous chunk's S0 and Y (both double buffered in LDS). Waves 8-11 ("loaders") stage
-// the operands and touch chunk c+3's lines so that the staging hits L2; only they ever wait for
-// global loads, so no compute wave stalls on load issue. A stage's k and q rows are read only
-// before the step's second barrier (the chain's Y phase, the output waves' operand copy), so the
-// loaders issue chunk c+2's k and q rows after that barrier and the rest of chunk c+1 after the
-// first: the ~60 KB a step passes through the CU's load path in both halves of the step.
+// Waves 0-3 ("chain") run the chain, waves 4-7 ("output") the output of the same chunk beside it.
+// Waves 8-11 ("loaders") stage the operands and touch chunk c+3's lines so that the staging hits L2;
+// only they ever wait for global loads, so no compute wave stalls on load issue.
+//
+// Barrier schedule: step c holds barriers A_c and B_c.
+//   before A_c   chain: S0 -> S0T; loaders: chunk c's Kh^T, P, V and table have landed
+//   A_c .. B_c   chain: S0T -> Y -> YT; output: S0T -> Q S0; both also read the operands they need
+//                after B_c (Kh^T; P and e^G). Loaders: issue Kh^T, P, V and table of chunk c+1, then
+//                wait for its k and q rows
+//   B_c .. A_c+1 chain: YT -> S1; output: YT -> O; both read chunk c+1's k (q) rows into registers.
+//                Loaders: issue the k and q rows of chunk c+2 (into the buffers of chunk c's, last read
+//                before A_c), then wait for the rest of chunk c+1
+// So each half of a step reads about the same from LDS, what the chain waits for after a barrier is S0T
+// or YT alone, and one buffer of each is enough, which is what lets 32 columns fit the LDS (a form with
+// the output a step behind the chain needed two). With 16 columns both forms take 160 us over 8192 tokens:
+// a step's chain alone takes about 0.7 us, its 60 KB of staging and the output's share of LDS and matrix
+// cores about 0.3 us each.
 // An f16 conv output (CoT = _Float16) gives q and k in place; from an f32 one they are the
 // prep's f16 rows in the record. V is read in place either way.
 constexpr int SCAN_THREADS = 768;
 
-template <typename CoT>
+template <typename CoT, int CW>
 __global__ __launch_bounds__(SCAN_THREADS) void gdn_chunk_scan(const char* __restrict__ scr, const CoT* __restrict__ co,
                                                       int cts, int nch, float* __restrict__ state, float* __restrict__ out,
                                                       int ots, int nt, int nv, int nk) {
+    constexpr int NCB = SD / CW;   // column blocks of the state per head
+    constexpr int NI = CW / 16;    // 16-column MFMA tiles per workgroup
     constexpr bool DIRECT = sizeof(CoT) == 2;
     constexpr size_t REC = rec_bytes<DIRECT>();
     constexpr int SP = SD + 8, VP = C + 8;
-    __shared__ __align__(16) ScanStage<CoT> B0;
-    __shared__ __align__(16) ScanStage<CoT> B1;
-    __shared__ __align__(16) _Float16 S0T[2][2][CW][SP];   // [chunk & 1][hi|lo][state column][key dim]
-    __shared__ __align__(16) _Float16 YT[2][2][CW][VP];    // [chunk & 1][hi|lo][state column][token]
-    __shared__ uint32_t PfSink[64];                         // landing words of the L2 touches, never read
+    typedef ScanStage<CoT, CW> Stage;
+    __shared__ __align__(16) Stage B0;
+    __shared__ __align__(16) Stage B1;
+    __shared__ __align__(16) _Float16 S0T[2][CW][SP];   // [hi|lo][state column][key dim]
+    __shared__ __align__(16) _Float16 YT[2][CW][VP];    // [hi|lo][state column][token]
+    __shared__ uint32_t PfSink[64];                      // landing words of the L2 touches, never read
 
     // XCD-aware placement: workgroups are dealt to the 8 XCDs round-robin by linear id, so id L
     // runs on XCD L % 8. All column blocks of one head go to the same XCD (head = xcd + 8*(slot/NCB))
@@ -487,29 +497,25 @@ __global__ __launch_bounds__(SCAN_THREADS) void gdn_chunk_scan(const char* __res
     auto vbase = [&](int cc) { return co + (size_t)cc * C * cts + 2 * nk * SD + h * SD + n0; };
     const int pitch = DIRECT ? cts : SD, koff = DIRECT ? nk * SD : C * SD;
     auto rows = [&](int cc) { return min(C, nt - cc * C); };
-    auto stage_kq = [&](int cc, ScanStage<CoT>& B, int part) {
-        scan_stage_kq<CoT>(qbase(cc), pitch, koff, rows(cc), B, part, l);
+    auto stage_kq = [&](int cc, Stage& B, int part) {
+        scan_stage_kq<CoT, CW>(qbase(cc), pitch, koff, rows(cc), B, part, l);
     };
-    auto stage_rest = [&](int cc, ScanStage<CoT>& B, int part) {
-        scan_stage_rest<CoT>(hrec + (size_t)cc * REC, vbase(cc), cts, rows(cc), B, part, l);
+    auto stage_rest = [&](int cc, Stage& B, int part) {
+        scan_stage_rest<CoT, CW>(hrec + (size_t)cc * REC, vbase(cc), cts, rows(cc), B, part, l);
     };
 
-    // Barrier schedule: step c (0 <= c <= nch) holds barriers A_c and B_c. The chain writes S0T[c&1]
-    // before A_c, reads stage c&1 and writes YT[c&1] between A_c and B_c, reads stage c&1's Kh^T and
-    // table after B_c. The output waves read S0T/YT[(c-1)&1] and stage c&1 between A_c and B_c. The
-    // loaders fill stage (c+1)&1's Kh^T, P, V and table after A_c and stage c&1's k and q rows (for
-    // chunk c+2) after B_c, and have chunk c+1 landed before A_{c+1}. Step nch only finishes the
-    // last chunk's output.
     if (wv >= 8) {
         const int part = wv - 8;
         constexpr int RL = (int)(REC / 128);                        // 128-byte lines of a record
         constexpr int QL = DIRECT ? 2 * C * (SD * 2 / 128) : 0;     // lines of the chunk's q and k rows
         constexpr int VLN = SD * (int)sizeof(CoT) / 128;            // lines of one V row of the head
-        // this block's share of chunk cc's 128-byte lines, 32 per loader wave (1024 per head): the
-        // record's, then (f16 conv output) those of the q and k rows, then those of the V rows
+        constexpr int TL = 1024 / (4 * NCB);                        // lines a loader wave touches (1024 per head)
+        static_assert(TL <= 64 && RL + QL + C * VLN <= 1024, "the touches cover a chunk's lines");
+        // this block's share of chunk cc's 128-byte lines: the record's, then (f16 conv output) those of
+        // the q and k rows, then those of the V rows
         auto touch = [&](int cc) {
             cc = min(cc, nch - 1);
-            const int u = cb * 128 + part * 32 + (l & 31), L = rows(cc);
+            const int u = cb * 4 * TL + part * TL + (l & (TL - 1)), L = rows(cc);
             const char* p = hrec + (size_t)cc * REC + 128 * min(u, RL - 1);
             if (u >= RL && u < RL + QL) {
                 const int v = u - RL, r = (v >> 1) & (C - 1);
@@ -520,6 +526,9 @@ __global__ __launch_bounds__(SCAN_THREADS) void gdn_chunk_scan(const char* __res
             }
             __builtin_amdgcn_global_load_lds((const void*)p, (lds_void*)PfSink, 4, 0, 0);
         };
+        // instructions of stage_rest this wave issues beyond those of parts 2 and 3 (at most 2)
+        constexpr int VN = scan_v_loads<CoT, CW>();
+        constexpr int REST = 6 + VN / 4;                              // parts 2 and 3 (VN is 2, 4 or 8)
         stage_kq(0, B0, part);
         stage_rest(0, B0, part);
         if (nch > 1) stage_kq(1, B1, part);
@@ -528,23 +537,32 @@ __global__ __launch_bounds__(SCAN_THREADS) void gdn_chunk_scan(const char* __res
         // chunk 0 landed; chunk 1's k and q rows and the touches may still be in flight
         if (nch > 1) IT_SCAN_WAIT_VMCNT(SCAN_KQ_LOADS + SCAN_TOUCH_AHEAD - 1);
         else IT_SCAN_WAIT_VMCNT(SCAN_TOUCH_AHEAD - 1);
-        for (int c = 0; c <= nch; ++c) {
+        lds_barrier();   // chunk 0 is there: the compute waves read its k (q) rows
+        for (int c = 0; c < nch; ++c) {
             lds_barrier();   // A_c
-            if (c + 1 < nch) stage_rest(c + 1, (c & 1) ? B0 : B1, part);
-            touch(c + SCAN_TOUCH_AHEAD);
-            lds_barrier();   // B_c
-            // chunk c+1 landed (its k and q rows went out a step earlier); the touch and chunk
-            // c+2's k and q rows may still be in flight
-            if (c + 2 < nch) {
-                stage_kq(c + 2, (c & 1) ? B1 : B0, part);
-                IT_SCAN_WAIT_VMCNT(SCAN_KQ_LOADS + 1);
-            } else {
-                IT_SCAN_WAIT_VMCNT(1);
+            if (c + 1 < nch) {
+                stage_rest(c + 1, (c & 1) ? B0 : B1, part);
+                // the k and q rows of chunk c+1 (issued a step ago, before the last touch) have landed;
+                // what is younger may still be in flight: the touch (two in step 0) and stage_rest's
+                if (part == 0) IT_SCAN_WAIT_VMCNT(REST + 1 + (VN % 4 > 0 ? 1 : 0) + 1);
+                else if (part == 1) IT_SCAN_WAIT_VMCNT(REST + (VN % 4 > 1 ? 1 : 0) + 1);
+                else IT_SCAN_WAIT_VMCNT(REST + 1);
             }
+            lds_barrier();   // B_c
+            // chunk c+1 landed; chunk c+2's k and q rows and the touch may still be in flight
+            if (c + 2 < nch) stage_kq(c + 2, (c & 1) ? B1 : B0, part);
+            touch(c + SCAN_TOUCH_AHEAD);
+            if (c + 2 < nch) IT_SCAN_WAIT_VMCNT(SCAN_KQ_LOADS + 1);
+            else IT_SCAN_WAIT_VMCNT(1);
         }
+        IT_SCAN_WAIT_VMCNT(0);   // the last touch lands in this workgroup's LDS
         return;
     }
     const int w = wv & 3;
+    const int rw = 16 * w + li;
+    // row rw (a token) of K or Q, dims 32ks + 8g ..; row r of Kh^T or P, tokens 32ks + 8g ..
+    auto row256 = [&](const _Float16* M, int ks) { return ld_h8(M + rw * SD + 8 * ((4 * ks + g) ^ swz256(rw))); };
+    auto row128 = [&](const _Float16* M, int r, int ks) { return ld_h8(M + r * C + 8 * ((4 * ks + g) ^ swz128(r))); };
     if (wv < 4) {
         float* sh = state + (size_t)h * SD * SD;
         // state slice in accumulator layout: st[mi][ni][i] = S[16(2w+mi) + 4g + i][n0 + 16ni + li]
@@ -555,82 +573,97 @@ __global__ __launch_bounds__(SCAN_THREADS) void gdn_chunk_scan(const char* __res
             for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) st[mi][ni][i] = sh[(size_t)(16 * (2 * w + mi) + 4 * g + i) * SD + n0 + 16 * ni + li];
-        const int rw = 16 * w + li;
-        for (int c = 0; c < nch; ++c) {
-            const int b = c & 1;
-            const ScanStage<CoT>& B = b ? B1 : B0;
+        h8 ka[4];
+        lds_barrier();   // chunk 0 is there
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) ka[ks] = row256(B0.K, ks);
+        auto step = [&](const Stage& B, const Stage& Bn, bool more) {
             // ---- S0 -> LDS as hi/lo, transposed to [column][key dim]
 #pragma unroll
             for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
-                for (int ni = 0; ni < NI; ++ni)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float v = st[mi][ni][i];
-                        const _Float16 hi = (_Float16)v, lo = (_Float16)(v - (float)hi);
-                        const int col = 16 * ni + li, dk = 16 * (2 * w + mi) + 4 * g + i;
-                        S0T[b][0][col][dk] = hi;
-                        S0T[b][1][col][dk] = lo;
-                    }
+                for (int ni = 0; ni < NI; ++ni) {
+                    h4 hi, lo;
+                    split_hi_lo4(st[mi][ni], hi, lo);
+                    *(h4*)&S0T[0][16 * ni + li][16 * (2 * w + mi) + 4 * g] = hi;
+                    *(h4*)&S0T[1][16 * ni + li][16 * (2 * w + mi) + 4 * g] = lo;
+                }
             lds_barrier();   // A_c
-            // ---- Y = V - e^G (K S0) for tokens 16w..16w+15 (k row 16w+li, dims 32ks+8g..). Every
-            // operand and V read is issued before the first product (the reads queue behind the
-            // loaders' LDS writes, so one round trip instead of one per product), the hi and lo
-            // products go to separate accumulators, and Y^T goes out as 8-byte pieces (tokens
-            // 16w + 4g + 0..3 of column li are contiguous).
-            static_assert(NI == 1, "one 16-column tile per workgroup");
-            h8 ka[4], sh[4], sl[4];
+            // ---- Y = V - e^G (K S0) for tokens 16w..16w+15; the hi and lo products go to separate
+            // accumulators, and Y^T goes out as 8-byte pieces (tokens 16w + 4g + 0..3 of a column)
+            h8 s0[NI][4], s1[NI][4];
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                ka[ks] = ld_h8(B.K + rw * SD + 8 * ((4 * ks + g) ^ swz256(rw)));
-                sh[ks] = ld_h8(&S0T[b][0][li][32 * ks + 8 * g]);
-                sl[ks] = ld_h8(&S0T[b][1][li][32 * ks + 8 * g]);
-            }
-            CoT vv[4];
+            for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) vv[i] = B.V[(16 * w + 4 * g + i) * CW + li];
+                for (int ni = 0; ni < NI; ++ni) {
+                    s0[ni][ks] = ld_h8(&S0T[0][16 * ni + li][32 * ks + 8 * g]);
+                    s1[ni][ks] = ld_h8(&S0T[1][16 * ni + li][32 * ks + 8 * g]);
+                }
+            CoT vv[NI][4];
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) vv[ni][i] = B.V[(16 * w + 4 * g + i) * CW + 16 * ni + li];
             const f4 eg = *(const f4*)&B.T[C + 16 * w + 4 * g];
-            f4 xh = {0.f, 0.f, 0.f, 0.f}, xl = {0.f, 0.f, 0.f, 0.f};
+            // Kh^T rows 16(2w+mi)+li, used after B_c
+            h8 kt[2][2];
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                xh = mfma16x16x32(ka[ks], sh[ks], xh);
-                xl = mfma16x16x32(ka[ks], sl[ks], xl);
-            }
-            h4 yh, yl;
+            for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float v = (float)vv[i] - eg[i] * (xh[i] + xl[i]);
-                yh[i] = (_Float16)v;
-                yl[i] = (_Float16)(v - (float)yh[i]);
-            }
-            *(h4*)&YT[b][0][li][16 * w + 4 * g] = yh;
-            *(h4*)&YT[b][1][li][16 * w + 4 * g] = yl;
-            lds_barrier();   // B_c
-            // ---- S1 = e^{G_last} S0 + Kh^T Y (Kh^T rows 16(2w+mi)+li, tokens 32ks+8g..), every
-            // operand read issued first
-            h8 kt[2][2], yv[2][2];
+                for (int mi = 0; mi < 2; ++mi) kt[ks][mi] = row128(B.KHT, 16 * (2 * w + mi) + li, ks);
+            const float gc = B.T[3 * C];
+            f4 xh[NI], xl[NI];
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
+            for (int ni = 0; ni < NI; ++ni) xh[ni] = xl[ni] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int mi = 0; mi < 2; ++mi) {
-                    const int rk = 16 * (2 * w + mi) + li;
-                    kt[ks][mi] = ld_h8(B.KHT + rk * C + 8 * ((4 * ks + g) ^ swz128(rk)));
+            for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+                for (int ni = 0; ni < NI; ++ni) {
+                    xh[ni] = mfma16x16x32(ka[ks], s0[ni][ks], xh[ni]);
+                    xl[ni] = mfma16x16x32(ka[ks], s1[ni][ks], xl[ni]);
                 }
 #pragma unroll
-                for (int hl = 0; hl < 2; ++hl) yv[ks][hl] = ld_h8(&YT[b][hl][li][32 * ks + 8 * g]);
-            }
-            const float gc = B.T[3 * C];
+            for (int ni = 0; ni < NI; ++ni) {
+                h4 yh, yl;
 #pragma unroll
-            for (int mi = 0; mi < 2; ++mi) st[mi][0] *= gc;
+                for (int i = 0; i < 4; ++i) {
+                    const float v = (float)vv[ni][i] - eg[i] * (xh[ni][i] + xl[ni][i]);
+                    yh[i] = (_Float16)v;
+                    yl[i] = (_Float16)(v - (float)yh[i]);
+                }
+                *(h4*)&YT[0][16 * ni + li][16 * w + 4 * g] = yh;
+                *(h4*)&YT[1][16 * ni + li][16 * w + 4 * g] = yl;
+            }
+            lds_barrier();   // B_c
+            // ---- S1 = e^{G_last} S0 + Kh^T Y; the next chunk's k rows on the way
+            h8 yv[NI][2][2];
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                    for (int hl = 0; hl < 2; ++hl) yv[ni][ks][hl] = ld_h8(&YT[hl][16 * ni + li][32 * ks + 8 * g]);
+            if (more) {
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks) ka[ks] = row256(Bn.K, ks);
+            }
+#pragma unroll
+            for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+                for (int ni = 0; ni < NI; ++ni) st[mi][ni] *= gc;
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
                 for (int hl = 0; hl < 2; ++hl)
 #pragma unroll
-                    for (int mi = 0; mi < 2; ++mi) st[mi][0] = mfma16x16x32(kt[ks][mi], yv[ks][hl], st[mi][0]);
+                    for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+                        for (int ni = 0; ni < NI; ++ni) st[mi][ni] = mfma16x16x32(kt[ks][mi], yv[ni][ks][hl], st[mi][ni]);
+        };
+        for (int c = 0; c < nch; c += 2) {
+            step(B0, B1, c + 1 < nch);
+            if (c + 1 < nch) step(B1, B0, c + 2 < nch);
         }
-        lds_barrier();   // A_nch
-        lds_barrier();   // B_nch
 #pragma unroll
         for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
@@ -639,73 +672,79 @@ __global__ __launch_bounds__(SCAN_THREADS) void gdn_chunk_scan(const char* __res
                 for (int i = 0; i < 4; ++i) sh[(size_t)(16 * (2 * w + mi) + 4 * g + i) * SD + n0 + 16 * ni + li] = st[mi][ni][i];
         return;
     }
-    // ---- output waves: O of chunk c-1 in step c, for tokens 16w..16w+15; the A operands of chunk
-    // c (q and P rows) and e^G of the output rows are copied from stage c&1 into registers in step
-    // c, used in step c+1
+    // ---- output waves: O = (e^G Q S0 + P Y) / sqrt(128) for tokens 16w..16w+15 of each chunk
     const float rs = 1.0f / sqrtf((float)SD);
-    const int rw = 16 * w + li;
-    h8 qg[4], pa[2];
-    f4 eg = {0.f, 0.f, 0.f, 0.f};
-    for (int c = 0; c <= nch; ++c) {
+    h8 qg[4];
+    lds_barrier();   // chunk 0 is there
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qg[ks] = row256(B0.Q, ks);
+    auto step = [&](const Stage& B, const Stage& Bn, int c, bool more) {
         lds_barrier();   // A_c
-        const int b = c & 1, pb = b ^ 1;
+        h8 s0[NI][4], s1[NI][4];
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni) {
+                s0[ni][ks] = ld_h8(&S0T[0][16 * ni + li][32 * ks + 8 * g]);
+                s1[ni][ks] = ld_h8(&S0T[1][16 * ni + li][32 * ks + 8 * g]);
+            }
+        h8 pa[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) pa[ks] = row128(B.P, rw, ks);
+        const f4 eg = *(const f4*)&B.T[C + 16 * w + 4 * g];   // e^{G_t} of rows 16w + 4g + i
+        f4 qh[NI], ql[NI];
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) qh[ni] = ql[ni] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni) {
+                qh[ni] = mfma16x16x32(qg[ks], s0[ni][ks], qh[ni]);
+                ql[ni] = mfma16x16x32(qg[ks], s1[ni][ks], ql[ni]);
+            }
         f4 oa[NI];
 #pragma unroll
-        for (int ni = 0; ni < NI; ++ni) oa[ni] = f4{0.f, 0.f, 0.f, 0.f};
-        if (c > 0) {
-            // every operand read first, then the products (hi and lo of S0 in separate accumulators)
-            h8 sh[4], sl[4], yv[2][2];
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                sh[ks] = ld_h8(&S0T[pb][0][li][32 * ks + 8 * g]);
-                sl[ks] = ld_h8(&S0T[pb][1][li][32 * ks + 8 * g]);
-            }
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                for (int hl = 0; hl < 2; ++hl) yv[ks][hl] = ld_h8(&YT[pb][hl][li][32 * ks + 8 * g]);
-            f4 qh = {0.f, 0.f, 0.f, 0.f}, ql = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                qh = mfma16x16x32(qg[ks], sh[ks], qh);
-                ql = mfma16x16x32(qg[ks], sl[ks], ql);
-            }
-            oa[0] = (qh + ql) * eg;   // e^{G_t} of rows 16w + 4g + i
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                for (int hl = 0; hl < 2; ++hl) oa[0] = mfma16x16x32(pa[ks], yv[ks][hl], oa[0]);
-        }
-        if (c < nch) {
-            // chunk c's operands, before B_c: the loaders overwrite stage c&1's q rows after it
-            const ScanStage<CoT>& B = b ? B1 : B0;
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) qg[ks] = ld_h8(B.Q + rw * SD + 8 * ((4 * ks + g) ^ swz256(rw)));
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) pa[ks] = ld_h8(B.P + rw * C + 8 * ((4 * ks + g) ^ swz128(rw)));
-            eg = *(const f4*)&B.T[C + 16 * w + 4 * g];
-        }
+        for (int ni = 0; ni < NI; ++ni) oa[ni] = (qh[ni] + ql[ni]) * eg;
         lds_barrier();   // B_c
-        if (c > 0) {
-            // (stores guarded per token only in a partial last chunk: per-lane conditions split
-            // the code into small blocks)
-            const int t0 = (c - 1) * C, L = min(C, nt - t0);
-            float* orow = out + (size_t)t0 * ots + (size_t)h * SD + n0 + li;
-            if (L == C) {
+        h8 yv[NI][2][2];
 #pragma unroll
-                for (int ni = 0; ni < NI; ++ni)
+        for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) orow[(size_t)(16 * w + 4 * g + i) * ots + 16 * ni] = oa[ni][i] * rs;
-            } else {
+            for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                for (int ni = 0; ni < NI; ++ni)
+                for (int hl = 0; hl < 2; ++hl) yv[ni][ks][hl] = ld_h8(&YT[hl][16 * ni + li][32 * ks + 8 * g]);
+        if (more) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int t = 16 * w + 4 * g + i;
-                        if (t < L) orow[(size_t)t * ots + 16 * ni] = oa[ni][i] * rs;
-                    }
-            }
+            for (int ks = 0; ks < 4; ++ks) qg[ks] = row256(Bn.Q, ks);
         }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int hl = 0; hl < 2; ++hl)
+#pragma unroll
+                for (int ni = 0; ni < NI; ++ni) oa[ni] = mfma16x16x32(pa[ks], yv[ni][ks][hl], oa[ni]);
+        // (stores guarded per token only in a partial last chunk: per-lane conditions split
+        // the code into small blocks)
+        const int t0 = c * C, L = min(C, nt - t0);
+        float* orow = out + (size_t)t0 * ots + (size_t)h * SD + n0 + li;
+        if (L == C) {
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) orow[(size_t)(16 * w + 4 * g + i) * ots + 16 * ni] = oa[ni][i] * rs;
+        } else {
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int t = 16 * w + 4 * g + i;
+                    if (t < L) orow[(size_t)t * ots + 16 * ni] = oa[ni][i] * rs;
+                }
+        }
+    };
+    for (int c = 0; c < nch; c += 2) {
+        step(B0, B1, c, c + 1 < nch);
+        if (c + 1 < nch) step(B1, B0, c + 1, c + 2 < nch);
     }
 }
 
@@ -720,9 +759,21 @@ hipError_t launch_gdn_chunked(const CoT* co, int cts, const float* br, const flo
                                                                   tail);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    // linear grid of 8 * NCB * ceil(nv / 8) workgroups, mapped to (head, column block) in-kernel
-    gdn_chunk_scan<CoT><<<dim3(8 * NCB * ((nv + 7) / 8)), SCAN_THREADS, 0, st>>>((const char*)scratch, co, cts, nch, state,
-                                                                                 out, ots, nt, nv, nk);
+    // State columns per scan workgroup. One workgroup fits a CU (its LDS) and a head's workgroups share an
+    // XCD of 32 CUs, so the scan takes ceil(heads per XCD x column blocks / 32) rounds of nch steps; a
+    // 32-column step takes 1.31 times a 16-column one (the k, q, Kh^T and P rows it stages and reads serve
+    // twice the columns). 48 V heads: two rounds of 16 columns or one of 32: layer at 500 tokens 42.4 against
+    // 37.7 us, 2000 122.8 against 109, 8192 504 against 438 us; 32 V heads (one round either way): 31.7
+    // against 34.8, 83 against 94, 304 against 354 us.
+    const int hx = (nv + 7) / 8;
+    const int r16 = (hx * (SD / 16) + 31) / 32, r32 = (hx * (SD / 32) + 31) / 32;
+    // linear grid of 8 x heads per XCD x column blocks workgroups, mapped to (head, column block) in-kernel
+    if (4 * r32 < 3 * r16)
+        gdn_chunk_scan<CoT, 32><<<dim3(8 * (SD / 32) * hx), SCAN_THREADS, 0, st>>>((const char*)scratch, co, cts, nch,
+                                                                                   state, out, ots, nt, nv, nk);
+    else
+        gdn_chunk_scan<CoT, 16><<<dim3(8 * (SD / 16) * hx), SCAN_THREADS, 0, st>>>((const char*)scratch, co, cts, nch,
+                                                                                   state, out, ots, nt, nv, nk);
     return hipGetLastError();
 }
 template hipError_t launch_gdn_chunked<float>(const float*, int, const float*, const float*, int, const float*,

@@ -493,3 +493,23 @@ def test_conv_runs_and_prefill_conv_state(dev, nt, nv, nk, K):
     ops.gdn_prefill(x, wd, st, dev_f32(d["beta_raw"], dev), dev_f32(d["alpha_raw"], dev), dev_f32(d["dt"], dev),
                     dev_f32(d["a"], dev), dev_f32(d["state"], dev), nv, nk)
     np.testing.assert_array_equal(host(st), wst)
+
+
+@pytest.mark.parametrize("nt,nv,nk", [(64, 40, 8), (65, 48, 16), (128, 64, 16), (193, 72, 24), (257, 33, 11)])
+def test_scan_column_blocks(dev, nt, nv, nk):
+    """Head counts whose scan takes 32 state columns a workgroup (more than 32 V heads), with one to five
+    chunks, whole and ragged, and head counts that leave an XCD short: the chunked scan and the
+    one-call prefill against the float64 recurrence on the conv output each consumed."""
+    announce(f"scan column blocks nt={nt} nv={nv} nk={nk}")
+    d = gdn_step_inputs(71 + nt, nt, nv=nv, nk=nk)
+    out, st = _chunked(dev, d, nv, nk)
+    o64, s64 = gdn_seq_f64(d["co"], d["beta_raw"], d["alpha_raw"], d["dt"], d["a"], d["state"], nv, nk)
+    assert np.abs(out - o64).max() <= OUT_TOL and np.abs(st - s64).max() <= STATE_TOL
+    d = gdn_inputs(81 + nt, nt=nt, nv=nv, nk=nk)
+    x, w = dev_f32(d["x"], dev), dev_f32(d["w"], dev)
+    co = ops.gdn_conv_l2norm(x, w, dev_f32(d["conv_state"], dev), 2 * nk).half().float()
+    st = dev_f32(d["state"], dev)
+    got = host(ops.gdn_prefill(x, w, dev_f32(d["conv_state"], dev), dev_f32(d["beta_raw"], dev),
+                               dev_f32(d["alpha_raw"], dev), dev_f32(d["dt"], dev), dev_f32(d["a"], dev), st, nv, nk))
+    o64, s64 = gdn_seq_f64(host(co), d["beta_raw"], d["alpha_raw"], d["dt"], d["a"], d["state"], nv, nk)
+    assert np.abs(got - o64).max() <= OUT_TOL and np.abs(host(st) - s64).max() <= STATE_TOL
