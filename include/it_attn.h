@@ -181,7 +181,8 @@ int it_attn_f16_mailbox(const float* q, int q_tok_stride, const uint16_t* kc, co
                         void* mailbox, size_t mailbox_bytes, void* scratch, size_t scratch_bytes, void* stream);
 
 /* The choice it_attn_f16 makes for this geometry and scratch budget: *kernel 1 (split-K) or 2
- * (flash), *chunk keys per split (0 = flash in one pass, no scratch), *bytes of scratch used.
+ * (flash), *chunk keys per split (0 = flash in one pass), *bytes of scratch it takes room for (flash
+ * may use less of it: longer splits, or one pass, where they are faster).
  * Returns nonzero if no split fits (only possible for nt < 16 with fewer than nt*nh*1040 bytes).
  * Scratch per split: the split-K kernel's records are 260 f32 words per (token, head); the flash
  * kernel's key-split records are 132 words per (token, head): {m, l, k, 0} and O as int16 in

@@ -84,7 +84,9 @@ size_t flash_scratch(int pos0, int nt, int nh, int chunk, bool f32rec = false) {
 // while nt*nh*ceil((pos0+nt)/C)*260 words exceed the room). The flash kernel ends at one pass over
 // all keys, which needs no scratch, so it always has a plan; the split-K kernel (nt < 16) can run
 // out of doublings only when even one record per (token, head) exceeds the budget. A chunk of 0
-// from the flash plan means the one-pass form. Returns false if nothing fits.
+// from the flash plan means the one-pass form. Returns false if nothing fits. `bytes` is the room of the
+// split so found; the flash kernel may run longer ranges in it, or one pass, where that is faster
+// (flash_run_chunk), and `chunk` is what it runs.
 struct AttnPlan { int kernel, chunk; size_t bytes; };
 bool plan_attn(int pos0, int nt, int nh, int nkv, int kernel, size_t budget, AttnPlan& p) {
     const long total = (long)pos0 + nt;
@@ -94,7 +96,7 @@ bool plan_attn(int pos0, int nt, int nh, int nkv, int kernel, size_t budget, Att
         const bool f32 = kernel == KERNEL_FLASH_F32;
         int c = flash_chunk(pos0, nt, nh, nkv, 0);
         while (c && flash_scratch(pos0, nt, nh, c, f32) > budget) c = (2L * c >= total) ? 0 : 2 * c;
-        p.chunk = c;
+        p.chunk = c ? it::flash_run_chunk(pos0, nt, nh, nkv, c) : 0;
         p.bytes = c ? flash_scratch(pos0, nt, nh, c, f32) : 0;
         return true;
     }

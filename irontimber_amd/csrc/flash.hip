@@ -3,29 +3,32 @@
 // counterparts are the multi-query split-K tiles of kernels/src/prefill_attention*.rs and
 // kernels/src/prefill_gqa.rs.
 //
-// Workgroup = 128 query rows sharing one KV head (rows r = t*G + g: token t, head g of the group,
-// G = nh/nkv). Per 64-key tile, in the transposed form so that every lane owns one query row:
+// Workgroup = 64 or 128 query rows sharing one KV head (rows r = t*G + g: token t, head g of the
+// group, G = nh/nkv). Per 64-key tile, in the transposed form so that every lane owns one query row:
 //   S^T  = K Q^T          A = K rows from LDS, B = q (f16, pre-scaled by scale*log2 e) held in
 //                         registers for the whole kernel
 //   softmax              running max / sum per query in the log2 domain, lane exchanges only
 //   O^T += V^T P^T        A = V^T through the LDS transpose read of the row-major V tile, B = P^T
 //                         straight from the S^T accumulator (f16); O^T stays in accumulators
-// K/V tiles go straight from HBM/L2 into double-buffered LDS (global_load_lds, 16 bytes per lane,
-// no registers): tile t+1 streams in while tile t is computed, one barrier per tile.
-// Two forms of the same tile:
-//   attn_flash_kernel     4 waves of 32 rows, 32x32x16 matrix ops, one wave per SIMD: each
-//                         transpose read of V serves 32 queries. One-pass launches of at least
-//                         a workgroup per CU (long prompts), which the LDS bytes per tile bound.
-//   attn_flash_w8_kernel  8 waves of 16 rows, 16x16x32 matrix ops, two waves per SIMD, so one
-//                         wave's softmax and waits overlap the other's matrix ops. Key-split
-//                         launches and short one-pass launches, bound by latency.
+// K/V tiles go straight from HBM/L2 into LDS (global_load_lds, 16 bytes per lane, no registers).
+// Three forms of the same tile:
+//   attn_flash_kernel       4 waves of 32 rows, 32x32x16 matrix ops, one wave per SIMD: each
+//                           transpose read of V serves 32 queries. Double-buffered tiles, one barrier
+//                           a tile. One-pass launches that fill the chip (long prompts, and shorter
+//                           ones after a long context), which the LDS bytes per tile bound.
+//   attn_flash_w_kernel<4>  4 waves of 16 rows, 16x16x32 matrix ops, one K and one V buffer (66 KB),
+//                           so two workgroups share a CU and 64 rows are the unit of work. One-pass
+//                           launches below that, and key-split ones of up to a workgroup per CU.
+//   attn_flash_w_kernel<8>  8 waves of 16 rows, two waves per SIMD on double-buffered tiles, so one
+//                           wave's softmax and waits overlap the other's matrix ops. The remaining
+//                           key-split launches.
 //
-// Key-split form (part != null, attn_flash_w8_kernel): workgroup (row tile, KV head, split s)
+// Key-split form (part != null, attn_flash_w_kernel): workgroup (row tile, KV head, split s)
 // covers keys [s*chunk, (s+1)*chunk) only and writes a partial record of each of its rows for the
 // merge kernel: the {m, l} of the decode partials (kernels/src/lib.rs:753-798) plus a scale k, and
 // O as int16 in units of k (FLASH_REC words a record: the O runs and the headers in two regions,
 // rec_index.h flash_o / flash_h). Used when one pass would leave most CUs idle: a 64-token
-// chunk after a long context has only 2 * ceil(64*G/128) row tiles.
+// chunk after a long context has only 2 * ceil(64*G/64) row tiles.
 #include "common.h"
 #include "internal.h"
 
@@ -33,7 +36,7 @@ namespace it {
 
 namespace {
 constexpr int HD = 256;
-constexpr int BM = 128, BN = 64, RW = 16;   // rows per workgroup, keys per tile, rows per wave
+constexpr int BM = 128, BN = 64, RW = 16;   // rows per workgroup (32-row form), keys per tile, rows per wave (w form)
 constexpr float RESCALE_SLACK = 8.0f;   // log2 units
 }
 
@@ -79,8 +82,8 @@ __device__ __forceinline__ void scale_acc(f16v& acc, float a) {
     }
 }
 
-// One pass over the keys (no records), for launches of at least a workgroup per CU, where each
-// V transpose read serving 32 queries keeps the tile below the LDS bound of the 16-row form.
+// One pass over the keys (no records), for launches that fill the chip, where each V transpose read
+// serving 32 queries keeps the tile below the LDS bound of the 16-row forms (launch_attn_flash).
 // QM: where the q operand comes from. 0: the f32 q rows, scaled and converted here. 2: q16,
 // pre-converted (q16[t][h][d] = f16(q * scale * log2 e), exactly what that conversion makes, from
 // it_attn_prep_f16_q16), half the bytes, read as whole rows and transposed through LDS as QM 0
@@ -100,8 +103,13 @@ __global__ __launch_bounds__(256) void attn_flash_kernel(
 
     const int G = nh / nkv, R = nt * G;
     const int nrt = (R + BM - 1) / BM;
-    const int rt = nrt - 1 - (int)blockIdx.x;          // heaviest row tile first
-    const int kh = blockIdx.y;
+    // Heaviest row tiles first. From three KV heads on the heads of a row tile lie side by side: head after
+    // head, the last one's heavy row tiles start when most of the launch is done (24/4 heads: 2048 tokens 98
+    // -> 76 us, 2500 125 -> 104, 4096 263 -> 254). With two heads or one, each heavy row tile is in the first
+    // round of 256 either way and head after head is up to 2 % faster after a context and at 5000 - 6000
+    // tokens, up to 2 % slower at 3500 - 4096.
+    const int id = blockIdx.x;
+    const int rt = nrt - 1 - (nkv > 2 ? id / nkv : id % nrt), kh = nkv > 2 ? id % nkv : id / nrt;
     // the wave index as a scalar: row counts, row walks and branches on them stay in SGPRs
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, hh = l >> 5, c = l & 31;
     const int r = rt * BM + 32 * w + c;                 // this lane's query row
@@ -363,7 +371,7 @@ __global__ __launch_bounds__(256) void attn_flash_kernel(
     }
 }
 
-// ---- eight waves of 16 query rows (16x16x32 matrix ops)
+// ---- waves of 16 query rows (16x16x32 matrix ops)
 // LDS tiles are unpadded 512-byte rows of 32 16-byte chunks; logical chunk j of row r lives at
 // physical chunk j ^ swz16(r) (swz16 < 16). A chunk's bank group is (chunk mod 16). The score reads
 // (one K row per lane, 16 lanes at a time) take rows that differ in bits 0, 1, 3 and 4, and the V
@@ -372,30 +380,68 @@ __global__ __launch_bounds__(256) void attn_flash_kernel(
 // distinct bank groups.
 __device__ __forceinline__ int swz16(int r) { return ((r & 3) << 1) | (((r >> 3) & 1) << 3) | ((r >> 4) & 1); }
 
-// Issue the direct-to-LDS loads of one 64-row tile: wave w moves rows 8w..8w+7, two rows (64 lanes
+// Issue the direct-to-LDS loads of one 64-row tile: wave w of NW moves 64 / NW rows, two rows (64 lanes
 // x 16 bytes) per instruction, each lane fetching the logical chunk that belongs at its physical
 // slot. Rows past kend-1 repeat row kend-1 (a tile issued past the end only refetches it).
 // Addresses are a uniform row base plus a 32-bit lane offset; the chunk part of the offsets (cj,
 // including the head's column) is computed once.
+template <int NW>
 __device__ __forceinline__ void tile_to_lds16(const uint16_t* __restrict__ src, int kvd, int kb, int kend,
-                                            const int (&cj)[4], _Float16* lds, int w, int l) {
+                                            const int (&cj)[32 / NW], _Float16* lds, int w, int l) {
     typedef __attribute__((address_space(3))) void lds_void;
     const int ts = min(kb, kend - 1);                      // first row of the tile, clamped
     const char* base = (const char*)(src + (size_t)ts * kvd);
     const int rmax = kend - 1 - ts;                        // >= 0
     const unsigned rowb = 2u * (unsigned)kvd;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = 8 * w + 2 * i + (l >> 5);
+    for (int i = 0; i < 32 / NW; ++i) {
+        const int r = 64 / NW * w + 2 * i + (l >> 5);
         const unsigned off = (unsigned)min(r, rmax) * rowb + (unsigned)cj[i];
-        __builtin_amdgcn_global_load_lds((const void*)(base + off), (lds_void*)(lds + (8 * w + 2 * i) * HD), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void*)(base + off), (lds_void*)(lds + (64 / NW * w + 2 * i) * HD), 16, 0, 0);
     }
 }
 
-// Two waves per SIMD (about 210 registers each), so one wave's softmax, waits and barrier overlap
+// First row tile (of bm rows) that sees any key of split k: the one whose last token is at k * chunk.
+__host__ __device__ __forceinline__ int flash_first_tile(int k, int chunk, int pos0, int G, int bm) {
+    const long d = (long)k * chunk - pos0;
+    return d > 0 ? (int)(d * G / bm) : 0;
+}
+
+// Workgroup id -> (row tile, KV head, split) of a key-split launch that holds only the row tiles which see keys
+// of the split. The KV heads of a row tile lie side by side, so that with two heads an XCD works on one of them
+// (head after head: 64 tokens at 4096 19.7 against 18.1 us, 24/4 heads 24.4 against 21.8).
+template <int NW>
+__device__ __forceinline__ void flash_split_job(int id, int nrt, int nkv, int pos0, int chunk, int G, int& rt, int& kh,
+                                                int& split) {
+    split = min(id / (nrt * nkv), pos0 / chunk);   // (the splits up to pos0's are seen by every row tile)
+    id -= split * nrt * nkv;
+    for (int n = nrt; id >= n * nkv; n = nrt - flash_first_tile(split, chunk, pos0, G, RW * NW)) {
+        id -= n * nkv;
+        ++split;
+    }
+    rt = nrt - 1 - id / nkv;
+    kh = id % nkv;
+}
+
+// Workgroup id -> (row tile, KV head) of a one-pass launch. Heaviest row tiles first. Two workgroups share a
+// CU and up to 512 are resident at once: ids 256 .. 511 take the rest in rising order, so that the lightest
+// shares with the heaviest.
+__device__ __forceinline__ void flash_job(int id, int nrt, int nkv, int& rt, int& kh) {
+    const int n = nrt * nkv, j = n > 256 && n <= 512 && id >= 256 ? n - 1 - (id - 256) : id;
+    rt = nrt - 1 - j / nkv;
+    kh = j % nkv;
+}
+
+// Two waves per SIMD (about 210 registers each), so one wave's softmax, waits and barriers overlap
 // the other's matrix ops; each V transpose read serves 16 queries, so a tile moves twice the LDS
-// bytes of the 32-row form. For key-split launches and one-pass launches of fewer workgroups than
-// CUs, which are bound by each workgroup's chain of dependent phases rather than by LDS.
+// bytes of the 32-row form. For launches bound by each workgroup's chain of dependent phases rather
+// than by LDS. The two waves of a SIMD belong to one workgroup of NW = 8 waves (128 rows, two K and two V
+// buffers, tile t+1 loading while t is computed, one barrier a tile) or to two workgroups of NW = 4 (64 rows
+// each, one K and one V buffer: V of a tile loads under its scores, K of the next under its P.V, two
+// barriers a tile). NW = 4 streams K and V once per 64 rows, but its wave alone on a SIMD takes 1.4
+// us a tile where eight take 1.8, short launches reach twice as many CUs, and two workgroups of
+// different length share a CU: one pass over 64 tokens 10.6 -> 8.4, 1024 tokens 40.8 -> 32.0, 1531 55.6
+// -> 44.2 us; key splits of 64 tokens at 1000 16.2 -> 13.9, at 8128 26.4 -> 24.8 us (NW = 8 -> 4).
 // F32REC: the key-split records in the split-K kernels' lossless f32 form instead ({m, l, 0, 0} +
 // O as 256 floats, 260 words, merged by the f32 combine), selectable through it_attn_f16_ex.
 // QM: where the q operand comes from. 0: the f32 q rows, scaled and converted here. 1 and 2: q16,
@@ -405,47 +451,59 @@ __device__ __forceinline__ void tile_to_lds16(const uint16_t* __restrict__ src, 
 // by every split from L2. 2 reads whole rows and transposes them through LDS as QM 0 does: for
 // one-pass launches, which read q once from memory, where a per-lane gather touches 16 rows per
 // instruction.
-template <bool F32REC, int QM>
-__global__ __launch_bounds__(512) void attn_flash_w8_kernel(
+template <int NW, bool F32REC, int QM>
+__global__ __launch_bounds__(64 * NW, 2) void attn_flash_w_kernel(
     const float* __restrict__ q, int qts, const _Float16* __restrict__ q16, int q16ts, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, int kvd, int pos0, int nh, int nkv, int nt, float scale, float* __restrict__ out,
     int ots, float* __restrict__ part, int chunk, int smax) {
-    // two K and two V buffers as distinct objects, so the compiler can tell that the loads
-    // streaming into one buffer never alias the reads of the other (no conservative waits)
+    static_assert(NW == 4 || (NW == 8 && QM != 2), "eight waves: key splits only");
+    constexpr bool DB = NW == 8;     // double-buffered tiles
+    const bool by_keys = NW == 8 || part != nullptr;   // key splits and records, or one pass
+    constexpr int BM = RW * NW;      // query rows per workgroup
+    // the K and V buffers as distinct objects, so the compiler can tell that the loads
+    // streaming into one buffer never alias the reads of another (no conservative waits)
     __shared__ __align__(16) _Float16 K0[BN * HD];
-    __shared__ __align__(16) _Float16 K1[BN * HD];
+    __shared__ __align__(16) _Float16 K1[DB ? BN * HD : 8];
     __shared__ __align__(16) _Float16 V0[BN * HD];
-    __shared__ __align__(16) _Float16 V1[BN * HD];
+    __shared__ __align__(16) _Float16 V1[DB ? BN * HD : 8];
 
     const int G = nh / nkv, R = nt * G;
     const int nrt = (R + BM - 1) / BM;
-    const int rt = nrt - 1 - (int)blockIdx.x;          // heaviest row tile first
-    const int kh = blockIdx.y;
+    int rt, kh, split = 0;
+    if (!by_keys) {
+        flash_job((int)blockIdx.x, nrt, nkv, rt, kh);
+    } else if (gridDim.y == 1) {
+        flash_split_job<NW>((int)blockIdx.x, nrt, nkv, pos0, chunk, G, rt, kh, split);
+    } else {
+        rt = nrt - 1 - (int)blockIdx.x / nkv;
+        kh = (int)blockIdx.x % nkv;
+        split = blockIdx.y;
+    }
     // the wave index as a scalar: row counts, row walks and branches on them stay in SGPRs
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, g = l >> 4, c = l & 15;
     const int r = rt * BM + RW * w + c;                 // this lane's query row
     const bool rvalid = r < R;
     const int t = rvalid ? r / G : 0;
     const int tmin = (rt * BM) / G, tmax = (min(R, rt * BM + BM) - 1) / G;
-    const int split = blockIdx.z;
-    const int kb0 = part ? split * chunk : 0;           // this workgroup's keys: [kb0, kend)
-    const int kend = part ? min(pos0 + tmax + 1, kb0 + chunk) : pos0 + tmax + 1;
+    const int kb0 = by_keys ? split * chunk : 0;        // this workgroup's keys: [kb0, kend)
+    const int kend = by_keys ? min(pos0 + tmax + 1, kb0 + chunk) : pos0 + tmax + 1;
     if (kb0 >= kend) return;                            // no row of the tile sees these keys
     const int kfull = pos0 + tmin + 1;                  // keys every row of the tile sees
     const int qlim = pos0 + t;                          // this row sees keys <= qlim
     const size_t head_off = (size_t)kh * HD;
 
     // byte offset of the logical chunk each lane's DMA slot holds, plus the KV head's column
-    int cj[4];
+    int cj[32 / NW];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) cj[i] = 2 * (int)head_off + 16 * ((l & 31) ^ swz16(8 * w + 2 * i + (l >> 5)));
+    for (int i = 0; i < 32 / NW; ++i) cj[i] = 2 * (int)head_off + 16 * ((l & 31) ^ swz16(64 / NW * w + 2 * i + (l >> 5)));
     // q as the B operand of S^T = K Q^T: lane (c, g) holds dims 32ks + 8g .. +7 of query row c,
     // scaled into log2 units. QM 0 and 2 read the wave's 16 rows whole and transpose them through
-    // the wave's own 8 KB of the second K/V buffers, which the first tile does not use (16-byte
-    // chunk index XOR row, so the operand reads of 16 rows hit distinct banks). The q loads go out
-    // before the first tile's, so the prologue costs one memory round trip.
+    // 8 KB of the second K/V buffers, which the first tile does not use, or (single buffers) of V's, the
+    // rows that this wave's own first V loads will fill (16-byte chunk index XOR row, so the operand
+    // reads of 16 rows hit distinct banks). The q loads go out before the first tile's, so the prologue
+    // costs one memory round trip.
     h8 qb[8];
-    _Float16* qs = (w < 4 ? K1 : V1) + (w & 3) * (RW * HD);
+    _Float16* qs = DB ? (w < 4 ? K1 : V1) + (w & 3) * (RW * HD) : V0 + w * (RW * HD);
     if constexpr (QM == 1) {
         const int rr = rvalid ? r : R - 1;
         const _Float16* qrow = q16 + (size_t)(rr / G) * q16ts + (size_t)(kh * G + rr % G) * HD + 8 * g;
@@ -454,8 +512,8 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
             const h8 v = ld_h8(qrow + 32 * ks);
             qb[ks] = rvalid ? v : h8{};
         }
-        tile_to_lds16(kc, kvd, kb0, kend, cj, K0, w, l);
-        tile_to_lds16(vc, kvd, kb0, kend, cj, V0, w, l);
+        tile_to_lds16<NW>(kc, kvd, kb0, kend, cj, K0, w, l);
+        if constexpr (DB) tile_to_lds16<NW>(vc, kvd, kb0, kend, cj, V0, w, l);
     } else if constexpr (QM == 2) {
         // two 512-byte rows per load instruction (lanes 0-31 row 2j, lanes 32-63 row 2j + 1 of the
         // wave's 16; rows past R zero)
@@ -478,8 +536,8 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
                 if (++go == G) { go = 0; ++to; }
             }
         }
-        tile_to_lds16(kc, kvd, kb0, kend, cj, K0, w, l);
-        tile_to_lds16(vc, kvd, kb0, kend, cj, V0, w, l);
+        tile_to_lds16<NW>(kc, kvd, kb0, kend, cj, K0, w, l);
+        if constexpr (DB) tile_to_lds16<NW>(vc, kvd, kb0, kend, cj, V0, w, l);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int i = 2 * j + hi;
@@ -502,8 +560,8 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
             qx[i] = ld_f4(src + 4 * l);
             if (++gq == G) { gq = 0; ++tq; }
         }
-        tile_to_lds16(kc, kvd, kb0, kend, cj, K0, w, l);
-        tile_to_lds16(vc, kvd, kb0, kend, cj, V0, w, l);
+        tile_to_lds16<NW>(kc, kvd, kb0, kend, cj, K0, w, l);
+        if constexpr (DB) tile_to_lds16<NW>(vc, kvd, kb0, kend, cj, V0, w, l);
         const float sc = scale * LOG2E;
 #pragma unroll
         for (int i = 0; i < RW; ++i) {
@@ -542,16 +600,9 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
         for (int d8 = 0; d8 < 8; ++d8) voff[d8] = rv * HD + 8 * ((2 * d8 + ((s & 3) >> 1)) ^ sw) + 4 * (s & 1);
     }
 
-    // one 64-key tile: K/V hold tile kb (issued one tile earlier); tile kb+BN streams into Kn/Vn
-    auto tile = [&](int kb, const _Float16* K, const _Float16* V, _Float16* Kn, _Float16* Vn) {
-        // tile kb has landed for this wave; after the barrier for every wave, and every wave is
-        // done with the buffers that tile kb+BN goes into
-        IT_WAIT_VMCNT(0);
-        __syncthreads();
-        // the next tile streams in while this one is computed; issued unconditionally (past the end
-        // it refetches row kend-1 into the idle buffers)
-        tile_to_lds16(kc, kvd, kb + BN, kend, cj, Kn, w, l);
-        tile_to_lds16(vc, kvd, kb + BN, kend, cj, Vn, w, l);
+    // ---- scores and softmax of the tile at kb, whose K rows are in K; P^T into pb
+    h8 pb[2];
+    auto scores = [&](int kb, const _Float16* K) {
         // ---- S^T = K Q^T, four 16-key blocks
         f4 sc[4];
 #pragma unroll
@@ -604,7 +655,6 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
         }
         const float msub = (m_run == -INFINITY) ? 0.0f : m_run;
         float lsum = 0.f;
-        h8 pb[2];
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -614,7 +664,9 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
                 pb[kk][j] = (_Float16)p;
             }
         l_run += lsum;   // this lane group's keys only; the groups are added after the loop
-        // ---- O^T += V^T P^T: step kk covers keys 32kk + 8g + 0..7 in lane group g
+    };
+    // ---- O^T += V^T P^T: step kk covers keys 32kk + 8g + 0..7 in lane group g
+    auto pv = [&](const _Float16* V) {
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -634,16 +686,45 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
     };
-    for (int kb = kb0; kb < kend; kb += 2 * BN) {
-        tile(kb, K0, V0, K1, V1);
-        if (kb + BN < kend) tile(kb + BN, K1, V1, K0, V0);
+    if constexpr (DB) {
+        // K/V hold tile kb (issued one tile earlier); tile kb+BN streams into Kn/Vn
+        auto tile = [&](int kb, const _Float16* K, const _Float16* V, _Float16* Kn, _Float16* Vn) {
+            // tile kb has landed for this wave; after the barrier for every wave, and every wave is
+            // done with the buffers that tile kb+BN goes into
+            IT_WAIT_VMCNT(0);
+            __syncthreads();
+            // the next tile streams in while this one is computed; issued unconditionally (past the end
+            // it refetches row kend-1 into the idle buffers)
+            tile_to_lds16<NW>(kc, kvd, kb + BN, kend, cj, Kn, w, l);
+            tile_to_lds16<NW>(vc, kvd, kb + BN, kend, cj, Vn, w, l);
+            scores(kb, K);
+            pv(V);
+        };
+        for (int kb = kb0; kb < kend; kb += 2 * BN) {
+            tile(kb, K0, V0, K1, V1);
+            if (kb + BN < kend) tile(kb + BN, K1, V1, K0, V0);
+        }
+        IT_WAIT_VMCNT(0);  // the loads issued past the end land in the buffers staged below
+    } else {
+        // one buffer each: V of a tile streams in under its scores and softmax, K of the next tile
+        // under its P.V (issued unconditionally, past the end it refetches row kend-1)
+        for (int kb = kb0; kb < kend; kb += BN) {
+            IT_WAIT_VMCNT(0);
+            __syncthreads();   // K of this tile is there, every wave is done with V (first tile: with its q rows)
+            tile_to_lds16<NW>(vc, kvd, kb, kend, cj, V0, w, l);
+            scores(kb, K0);
+            IT_WAIT_VMCNT(0);
+            __syncthreads();   // V of this tile is there, every wave is done with K
+            tile_to_lds16<NW>(kc, kvd, kb + BN, kend, cj, K0, w, l);
+            pv(V0);
+        }
+        IT_WAIT_VMCNT(0);
     }
     // ---- epilogue. Lane (c, g) holds O^T of query c at dims 16db + 4g + 0..3; wave w stages its
     // 16 rows x 256 f32 in its own 16 KB of the tile buffers (16-byte chunk index XOR row,
     // conflict-free), then writes whole rows: one 1 KB row per store instruction.
-    IT_WAIT_VMCNT(0);  // the loads issued past the end land in the buffers staged below
     __syncthreads();   // every wave is done with the last tile
-    float* os = (float*)(w < 2 ? K0 : w < 4 ? K1 : w < 6 ? V0 : V1) + (w & 1) * (RW * HD);
+    float* os = (float*)(DB ? (w < 2 ? K0 : w < 4 ? K1 : w < 6 ? V0 : V1) : (w < 2 ? K0 : V0)) + (w & 1) * (RW * HD);
     // max |O| over the lane's 64 dims of its row (the int16 record scale), taken on the bit
     // patterns of |O|: NaN patterns sort above infinity, so a NaN or infinite O (from a NaN or
     // infinite V) reaches the record's scale and the merged output instead of being quantised
@@ -659,7 +740,7 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
             abits = b > abits ? b : abits;
         }
     }
-    __shared__ __align__(16) float ml[8][3][RW];   // per wave: running max, sum and max |O| of its 16 queries
+    __shared__ __align__(16) float ml[NW][3][RW];   // per wave: running max, sum and max |O| of its 16 queries
     l_run = sum_xor32(sum_xor16(l_run));
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -673,7 +754,7 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
     const int rw = __builtin_amdgcn_readfirstlane(rt * BM + RW * w);
     const int nrow = min(RW, R - rw);
     int tq = __builtin_amdgcn_readfirstlane(rw / G), gq = rw - tq * G;   // (token, q-head) of row rw + i
-    if (F32REC && part) {
+    if (F32REC && by_keys) {
         // f32 records of (token, head, split), 260 words each: {m, l, 0, 0}, then O
         if (l < nrow) {
             const int tl = (rw + l) / G, gl = rw + l - tl * G;
@@ -689,7 +770,7 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
         }
         return;
     }
-    if (part) {
+    if (by_keys) {
         // partial records of (token, head, split), FLASH_REC words each: O as 256 int16 in a
         // 512-byte run of its own (whole cache lines: no line is shared with another split's
         // record, which another workgroup writes), the header in a packed region: {m, l, k, 0} with m in
@@ -723,7 +804,7 @@ __global__ __launch_bounds__(512) void attn_flash_w8_kernel(
             __builtin_nontemporal_store(pk, dst + l);
             if (++gq == G) { gq = 0; ridx += rnext; } else { ridx += smax; }
         };
-        // a full 16-row wave (every wave when the row count is a multiple of 128) runs the rows
+        // a full 16-row wave (every wave when the row count is a multiple of 16 NW) runs the rows
         // as one straight block, so their conversions and stores interleave
         if (nrow == RW) {
 #pragma unroll
@@ -757,74 +838,151 @@ hipError_t launch_attn_flash(const float* q, int qts, const uint16_t* kc, const 
                              int nh, int nkv, int nt, float scale, float* out, int ots, hipStream_t st,
                              const uint16_t* q16, int q16ts) {
     const int R = nt * (nh / nkv);
-    const dim3 grid((R + BM - 1) / BM, nkv);
+    const unsigned n32 = (unsigned)((R + BM - 1) / BM * nkv), n16 = (unsigned)((R + 4 * RW - 1) / (4 * RW) * nkv);
     const _Float16* qh = (const _Float16*)q16;
-    // a workgroup per CU or more: the 32-row form (at 8192 tokens 4-6 % faster; below ~128
-    // workgroups the 16-row form, e.g. 64 tokens 14.1 -> 10.6 us)
-    if (grid.x * grid.y >= 256) {
-        if (q16)
-            attn_flash_kernel<2><<<grid, 256, 0, st>>>(q, qts, qh, q16ts, kc, vc, kvd, pos0, nh, nkv, nt, scale, out, ots);
-        else
-            attn_flash_kernel<0><<<grid, 256, 0, st>>>(q, qts, qh, q16ts, kc, vc, kvd, pos0, nh, nkv, nt, scale, out, ots);
-    } else if (q16) {
-        attn_flash_w8_kernel<false, 2><<<grid, 512, 0, st>>>(q, qts, qh, q16ts, kc, vc, kvd, pos0, nh, nkv, nt, scale,
-                                                             out, ots, nullptr, 0, 1);
+    // 16-row form (64 rows a workgroup, up to two a CU) or 32-row form (128 rows, one a CU). The former:
+    //  - up to 256 workgroups of its own, each alone on its CU (1024 tokens at 7000: 189 against 218 us);
+    //  - up to 512, when the rows' own keys are at least 2/5 of all: the two workgroups of a CU are
+    //    then of different length (16/2 heads, 2000 tokens at 1000 and 2000: 94 against 100 and 129 against
+    //    134 us; 1024 at 3000: 105 against 117). With a longer context both are long and the LDS bytes
+    //    bound them (1280 at 6000: 218 against 200; 24/4 heads, 900 at 6000: 218 against 190);
+    //  - up to 2/3 of two rounds of 512 when there is next to no context: 2300 and 2600 tokens 79 and 90
+    //    against 83 and 94 us, 24/4 heads 1800 63 against 66. Beyond, or with a context, slower: 3000
+    //    tokens 111 against 107, 24/4 heads 2048 81 against 76, 1600 at 1000 116 against 104.
+    const bool w16 = n16 <= 256 || (n16 <= 512 && 2L * pos0 <= 3L * nt) || (n16 <= 682 && 8L * pos0 <= nt);
+#define IT_FLASH(K_, N_)                                                                                               \
+    K_<<<N_, 256, 0, st>>>(q, qts, qh, q16ts, kc, vc, kvd, pos0, nh, nkv, nt, scale, out, ots IT_FLASH_TAIL)
+    if (w16) {
+#define IT_FLASH_TAIL , nullptr, 0, 1
+        if (q16) IT_FLASH((attn_flash_w_kernel<4, false, 2>), n16);
+        else IT_FLASH((attn_flash_w_kernel<4, false, 0>), n16);
+#undef IT_FLASH_TAIL
     } else {
-        attn_flash_w8_kernel<false, 0><<<grid, 512, 0, st>>>(q, qts, qh, q16ts, kc, vc, kvd, pos0, nh, nkv, nt, scale,
-                                                             out, ots, nullptr, 0, 1);
+#define IT_FLASH_TAIL
+        if (q16) IT_FLASH(attn_flash_kernel<2>, n32);
+        else IT_FLASH(attn_flash_kernel<0>, n32);
+#undef IT_FLASH_TAIL
     }
+#undef IT_FLASH
     return hipGetLastError();
 }
 
-// Keys per split of a launch that one pass would leave short of workgroups (fewer than 128), 0 for one
-// pass. One workgroup fits a CU, so a launch takes whole rounds of 256 workgroups, each as long as its
-// longest split: the split minimises
+// Workgroups of `bm` rows that have keys to see when the keys are split into ranges of `chunk`.
+static long flash_split_wgs(int pos0, int nt, int G, int nkv, int bm, int chunk) {
+    const int nrt = (int)(((long)nt * G + bm - 1) / bm), splits = (int)(((long)pos0 + nt + chunk - 1) / chunk);
+    const int all = pos0 / chunk + 1;   // splits that every row sees
+    long n = (long)nrt * min(all, splits);
+    for (int k = all; k < splits; ++k) n += nrt - flash_first_tile(k, chunk, pos0, G, bm);
+    return n * nkv;
+}
+
+// Ranges to weigh: `keys` in smax .. 2 equal ones, or up to two tiles longer ones, of at least `least` keys. A
+// short last range is seen by fewer row tiles, which can save a round (700 tokens at 1500: three ranges of 768
+// keys make 260 workgroups, of 832 244).
+template <class F>
+static void flash_ranges(int keys, int least, int smax, F&& weigh) {
+    for (int s = smax, last = 0; s >= 2; --s) {
+        const int c0 = max(((keys + s - 1) / s + BN - 1) / BN * BN, least);
+        for (int c = max(c0, last + BN); c <= c0 + 2 * BN && c < keys; c += BN) {
+            last = c;
+            weigh(c);
+        }
+    }
+}
+
+// A key-split launch in 64-row workgroups (NW = 4)? Up to one per CU of them: at one chunk always faster than
+// half as many of 128 rows (16 tokens at 1000 13.7 -> 11.7 us, 64 at 4096 21.3 -> 19.3, 128 at 8000 35.2
+// -> 34.9); two to a CU they only equal 128 rows.
+static bool flash_split_w4(int pos0, int nt, int G, int nkv, int chunk) {
+    return flash_split_wgs(pos0, nt, G, nkv, 4 * RW, chunk) <= 256;
+}
+
+// Keys per split that the records of a prompt call are given room for, when one pass would leave it short of
+// workgroups (fewer than 128 of 128 rows); 0 for one pass. A launch takes whole rounds of 256 workgroups of 128
+// rows, each as long as its longest split: the split minimises
 //   rounds * (1.8 us a 64-key tile + 12 us a workgroup) + 1 us per 32 workgroups of records to merge
 // over the splits into 1 .. 32 ranges (what the row merge holds: 24 tokens at 8000 in 63 ranges 24.4, in 32
-// 21.2 us), counting the workgroups that have keys to see.
-// The split that reaches 256 workgroups without regard to the rounds, which this rule replaces, left a
-// second round of a few workgroups at most sizes: 441 tokens at position 7560 (280 workgroups) 110 against
-// 77 us, 24/4 heads with 64 tokens at 4096 34 against 26 us, 256 at 5000 75 against 49 us, 512 at 5000
-// 132 against 99 us; where it had met a whole round (16/2 heads, 64 and 512 tokens) the choice is the same.
+// 21.2 us), counting the workgroups that have keys to see. The launch itself may take longer ranges
+// (flash_run_chunk).
+// The split that reaches 256 workgroups without regard to the rounds left a second round of a few workgroups
+// at most sizes: 441 tokens at position 7560 (280 workgroups) 107 against 80 us, 24/4 heads with 64
+// tokens at 4096 34 against 26 us, 256 at 5000 75 against 49 us, 512 at 5000 132 against 99 us; where it had
+// met a whole round (16/2 heads, 64 and 512 tokens) the choice is the same.
 int flash_split_chunk(int pos0, int nt, int nh, int nkv) {
-    const int G = nh / nkv, R = nt * G, nrt = (R + BM - 1) / BM, wgs = nrt * nkv;
+    const int G = nh / nkv, R = nt * G, wgs = (R + BM - 1) / BM * nkv;
     const int keys = pos0 + nt;
     if (wgs >= 128 || keys <= 4 * BN) return 0;
     const int smax = wgs <= 64 ? 32 : (2 * 256 + wgs - 1) / wgs;   // (beyond: always more rounds)
-    long best_cost = -1;
+    long best_cost = (long)(wgs + 255) / 256 * (288L * ((keys + BN - 1) / BN) + 1920);   // one pass; 1/160 us
     int best = 0;
-    for (int s = 1; s <= smax; ++s) {
-        const int c = ((keys + s - 1) / s + BN - 1) / BN * BN;
-        if (c == best) continue;
-        long n = 0;
-        for (int rt = 0; rt < nrt; ++rt) n += (pos0 + (min(R, rt * BM + BM) - 1) / G + c) / c;   // ceil(keys seen / c)
-        n *= nkv;
-        const long cost = (n + 255) / 256 * (288L * (c / BN) + 1920) + (s > 1 ? 5 * n : 0);   // 1/160 us
-        if (best_cost < 0 || cost < best_cost) {
+    flash_ranges(keys, BN, smax, [&](int c) {
+        const long n = flash_split_wgs(pos0, nt, G, nkv, BM, c);
+        const long cost = (n + 255) / 256 * (288L * (c / BN) + 1920) + 5 * n;
+        if (cost <= best_cost) {
             best_cost = cost;
             best = c;
         }
-    }
-    return best >= keys ? 0 : best;
+    });
+    return best;
+}
+
+// Keys per split that a launch with room for splits of `chunk` keys takes: ranges as long or longer, or 0 for
+// one pass, whichever is fastest by
+//   up to 256 workgroups of 64 rows   1.4 us a 64-key tile + 9 us
+//   else workgroups of 128 rows       rounds of 256 * (1.9 us a tile + 9 us)
+//                                     both + 1 us per 4096 record rows and 1 us per 2048 output rows to merge
+//   one pass, 64 rows                 1.4 us a tile + 8.5 us
+// Over 586 splits of 16 .. 1000 tokens at 0 .. 7500, 16/2 and 24/4 heads, the choice by these costs is on
+// average 0.3 % slower than the fastest measured one. At the room's own split and at the choice: 64 tokens at
+// 4096 (22 ranges, 13) 19.4 and 17.6 us, at 1000 14.6 and 12.2, 16 at 8000 19.3 and 16.0, 24/4 heads 64 at 4096
+// 26 and 21.5, 300 at 0 (one pass) 17.4 and 14.5, 1000 at 0 (one pass) 36.6 and 30.5.
+int flash_run_chunk(int pos0, int nt, int nh, int nkv, int chunk) {
+    const int G = nh / nkv, keys = pos0 + nt;
+    long best_cost = 224L * ((keys + BN - 1) / BN) + 1360;   // 1/160 us
+    int best = 0;
+    flash_ranges(keys, chunk, (keys + chunk - 1) / chunk, [&](int c) {
+        const long n4 = flash_split_wgs(pos0, nt, G, nkv, 4 * RW, c);
+        long cost = 224L * (c / BN) + 1440 + 5 * n4 / 2;
+        if (n4 > 256) {
+            const long n8 = flash_split_wgs(pos0, nt, G, nkv, 8 * RW, c);
+            cost = (n8 + 255) / 256 * (304L * (c / BN) + 1440) + 5 * n8;
+        }
+        cost += 5L * nt * nh / 64;
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = c;
+        }
+    });
+    return best;
 }
 
 hipError_t launch_attn_flash_split(const float* q, int qts, const uint16_t* kc, const uint16_t* vc, int kvd, int pos0,
                                    int nh, int nkv, int nt, float scale, float* out, int ots, float* part, int chunk,
                                    hipStream_t st, bool f32rec, const uint16_t* q16, int q16ts) {
-    const int R = nt * (nh / nkv);
     const int smax = idx::split_count((long)pos0 + nt, chunk);
-    const dim3 grid((R + BM - 1) / BM, nkv, smax);
+    const int nw = flash_split_w4(pos0, nt, nh / nkv, nkv, chunk) ? 4 : 8;
+    // One workgroup per (row tile, KV head) and split. Where that is more than the CUs, only those with keys: the
+    // others leave at once, but each holds a CU until then and the rest are spread unevenly behind them (850
+    // tokens at 0 in ranges of 256, 432 workgroups, 240 of them with keys: 38.8 -> 30.7 us; below 256 finding
+    // its split costs a workgroup 0.4 - 0.7 us: 64 tokens at 4096 17.4 -> 18.1).
+    const int nrt = (nt * (nh / nkv) + nw * RW - 1) / (nw * RW);
+    const dim3 grid = (long)nrt * nkv * smax <= 256
+                          ? dim3(nrt * nkv, smax)
+                          : dim3((unsigned)flash_split_wgs(pos0, nt, nh / nkv, nkv, nw * RW, chunk));
     const _Float16* qh = (const _Float16*)q16;
-#define IT_FLASH_SPLIT(F32_, Q16_)                                                                                     \
-    attn_flash_w8_kernel<F32_, Q16_><<<grid, 512, 0, st>>>(q, qts, qh, q16ts, kc, vc, kvd, pos0, nh, nkv, nt, scale, out, \
-                                                        ots, part, chunk, smax)
+#define IT_FLASH_SPLIT(NW_, F32_, Q16_)                                                                                \
+    attn_flash_w_kernel<NW_, F32_, Q16_><<<grid, 64 * NW_, 0, st>>>(q, qts, qh, q16ts, kc, vc, kvd, pos0, nh, nkv, nt,  \
+                                                                    scale, out, ots, part, chunk, smax)
+#define IT_FLASH_SPLIT_N(F32_, Q16_)                                                                                   \
+    (nw == 4 ? IT_FLASH_SPLIT(4, F32_, Q16_) : IT_FLASH_SPLIT(8, F32_, Q16_))
     if (f32rec) {
-        if (q16) IT_FLASH_SPLIT(true, 1);
-        else IT_FLASH_SPLIT(true, 0);
+        if (q16) IT_FLASH_SPLIT_N(true, 1);
+        else IT_FLASH_SPLIT_N(true, 0);
     } else {
-        if (q16) IT_FLASH_SPLIT(false, 1);
-        else IT_FLASH_SPLIT(false, 0);
+        if (q16) IT_FLASH_SPLIT_N(false, 1);
+        else IT_FLASH_SPLIT_N(false, 0);
     }
+#undef IT_FLASH_SPLIT_N
 #undef IT_FLASH_SPLIT
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -211,12 +211,15 @@ def test_plan_fits_reference_room_sweep(tmp_path, nh, nkv):
                                             (5000, 256, 24, 4), (5000, 512, 24, 4), (7680, 512, 16, 2),
                                             (8000, 24, 16, 2), (1000, 16, 16, 2)])
 def test_flash_split_fills_whole_rounds(pos0, nt, nh, nkv):
-    """Key splits of prompt chunks: at most 256 workgroups (one round of one a CU), at least half of
-    them where there are keys enough, at most the 32 records a row that the row merge holds."""
+    """Key splits of prompt chunks: at most 256 workgroups of 64 or else of 128 rows with keys to see (one round
+    of one a CU), at least half of them where there are keys enough, at most the 32 records a row that the
+    row merge holds."""
     rc, kernel, chunk, _ = plan(pos0, nt, nh, nkv, 1 << 40)
     assert (rc, kernel) == (0, 2) and chunk % 64 == 0 and 0 < chunk < pos0 + nt
-    splits = -(-(pos0 + nt) // chunk)
-    wgs = -(-nt * (nh // nkv) // 128) * nkv * splits
+    splits, g = -(-(pos0 + nt) // chunk), nh // nkv
+    w64, w128 = (nkv * sum(-(-(pos0 + -(-min(r0 + rows, nt * g) // g)) // chunk) for r0 in range(0, nt * g, rows))
+                 for rows in (64, 128))   # splits up to each row tile's last token
+    wgs = w64 if w64 <= 256 else w128
     assert wgs <= 256 and splits <= 32 and (wgs > 128 or splits >= 16)
 
 

@@ -161,6 +161,37 @@ def test_flash_split_plans(dev, ctx, nt, nh, nkv):
     assert np.isfinite(got).all() and np.abs(got - want).max() <= TOL
 
 
+@pytest.mark.parametrize("ctx,nt,nh,nkv", [(8, 8, 16, 2), (9, 9, 16, 2), (12, 11, 24, 4), (129, 65, 16, 2),
+                                           (1025, 1025, 16, 2), (1400, 1400, 24, 4), (2100, 2100, 16, 2),
+                                           (3100, 3100, 16, 2), (2300, 1030, 16, 2), (2100, 2100, 24, 4)])
+def test_flash_64_row_one_pass(dev, ctx, nt, nh, nkv):
+    """One pass in workgroups of 64 rows (16-row waves): a wave, a tile and one past it, two workgroups a CU in
+    both orders of their launch, and past its range (three heads and more, two heads), with f32 and with
+    pre-converted q, against the oracle."""
+    q, kb, vb = attn_inputs(67, ctx=ctx, nt=nt, nh=nh, nkv=nkv)
+    announce(f"flash one pass {ctx} {nt} {nh}/{nkv}")
+    qd, kc, vc = dev_f32(q.reshape(nt, -1), dev), dev_f16bits(kb, dev), dev_f16bits(vb, dev)
+    qh = (qd.view(nt, nh, 512)[:, :, :256] * (256 ** -0.5 * 1.4426950408889634)).half().reshape(nt, -1).contiguous()
+    scr = torch.empty(16, dtype=torch.uint8, device=dev)   # no room for records
+    outs = [host(ops.attn_f16(qd, kc, vc, ctx - nt, nh, nkv, kernel=ops.KERNEL_FLASH, scratch=scr))]
+    if nt >= 16:   # (fewer tokens with pre-converted q take the split-K kernels)
+        outs.append(host(ops.attn_f16_q16(qd, qh, kc, vc, ctx - nt, nh, nkv, scratch=scr)))
+    for t0 in sorted({0, max(0, nt // 2 - 8), max(0, nt - 16)}):
+        n = min(16, nt - t0)
+        want = oracle.attn(q[t0:t0 + n].reshape(n, -1), kb, vb, ctx - nt + t0, nh, nkv)
+        for got in outs:
+            assert np.isfinite(got).all() and np.abs(got[t0:t0 + n] - want).max() <= TOL
+
+
+@pytest.mark.parametrize("nt,pos0,chunk", [(1, 700, 64), (9, 700, 128), (64, 4096, 320), (64, 4096, 256), (130, 500, 64)])
+@pytest.mark.parametrize("kernel", [ops.KERNEL_FLASH, ops.KERNEL_FLASH_F32])
+def test_flash_split_workgroup_rows(dev, nt, pos0, chunk, kernel):
+    """Key splits in workgroups of 64 rows (up to 256 of them) and of 128, ragged row tiles and key ranges,
+    both record forms, against the oracle."""
+    got, want = run_case(dev, 71, pos0 + nt, nt, kernel=kernel, chunk=chunk)
+    assert np.isfinite(got).all() and np.abs(got - want).max() <= TOL
+
+
 @pytest.mark.parametrize("chunk", [0, 64, 192, 640])
 def test_flash_f32_records(dev, chunk):
     """The key-split flash path with lossless f32 records (kernel 3: the split-K kernels' 260-word
