@@ -928,12 +928,12 @@ int flash_split_chunk(int pos0, int nt, int nh, int nkv) {
 
 // Keys per split that a launch with room for splits of `chunk` keys takes: ranges as long or longer, or 0 for
 // one pass, whichever is fastest by
-//   up to 256 workgroups of 64 rows   1.4 us a 64-key tile + 9 us
+//   up to 256 workgroups of 64 rows   1.4 us a 64-key tile + 8.5 us
 //   else workgroups of 128 rows       rounds of 256 * (1.9 us a tile + 9 us)
 //                                     both + 1 us per 4096 record rows and 1 us per 2048 output rows to merge
 //   one pass, 64 rows                 1.4 us a tile + 8.5 us
-// Over 586 splits of 16 .. 1000 tokens at 0 .. 7500, 16/2 and 24/4 heads, the choice by these costs is on
-// average 0.3 % slower than the fastest measured one. At the room's own split and at the choice: 64 tokens at
+// Over 773 splits of 16 .. 1000 tokens at 0 .. 7200, 16/2 and 24/4 heads, the choice by these costs is on
+// average 0.2 % slower than the fastest measured one. At the room's own split and at the choice: 64 tokens at
 // 4096 (22 ranges, 13) 19.4 and 17.6 us, at 1000 14.6 and 12.2, 16 at 8000 19.3 and 16.0, 24/4 heads 64 at 4096
 // 26 and 21.5, 300 at 0 (one pass) 17.4 and 14.5, 1000 at 0 (one pass) 36.6 and 30.5.
 int flash_run_chunk(int pos0, int nt, int nh, int nkv, int chunk) {
@@ -942,7 +942,7 @@ int flash_run_chunk(int pos0, int nt, int nh, int nkv, int chunk) {
     int best = 0;
     flash_ranges(keys, chunk, (keys + chunk - 1) / chunk, [&](int c) {
         const long n4 = flash_split_wgs(pos0, nt, G, nkv, 4 * RW, c);
-        long cost = 224L * (c / BN) + 1440 + 5 * n4 / 2;
+        long cost = 224L * (c / BN) + 1360 + 5 * n4 / 2;
         if (n4 > 256) {
             const long n8 = flash_split_wgs(pos0, nt, G, nkv, 8 * RW, c);
             cost = (n8 + 255) / 256 * (304L * (c / BN) + 1440) + 5 * n8;
