@@ -223,6 +223,18 @@ def test_flash_split_fills_whole_rounds(pos0, nt, nh, nkv):
     assert wgs <= 256 and splits <= 32 and (wgs > 128 or splits >= 16)
 
 
+def test_misaligned_scratch_refused_where_room_is_planned():
+    """A prompt call whose plan takes room for records refuses a misaligned scratch, also where the
+    launch itself would be one pass (the pointers are never dereferenced)."""
+    lib, fake = _lib.lib(), ctypes.c_void_p(1 << 20)
+    for pos0, nt, one_pass in ((0, 300, True), (4096, 64, False)):
+        rc, kernel, chunk, room = plan(pos0, nt, 16, 2, 1 << 40)
+        assert (rc, kernel, chunk == 0) == (0, 2, one_pass) and room > 0
+        assert lib.it_attn_f16(fake, 16 * 512, fake, fake, 512, pos0, 256, 16, 2, nt, 0.0625, fake, 16 * 256,
+                               ctypes.c_void_p((1 << 20) + 4), room, None) != 0
+        assert "aligned" in _lib.last_error()
+
+
 def plan(pos0, nt, nh, nkv, budget):
     k, c, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
     rc = _lib.lib().it_attn_plan(pos0, nt, 256, nh, nkv, budget, ctypes.byref(k), ctypes.byref(c), ctypes.byref(b))
