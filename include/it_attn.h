@@ -73,7 +73,10 @@ int it_attn_prep_f16_q16(float* q, int q_tok_stride, const float* k, const float
                          int sec2, int sec3, int round_mode, uint16_t* q16, int q16_tok_stride, float scale,
                          void* stream);
 
-/* Bytes of scratch it_attn_f16 needs for this call geometry (0 if the chosen kernel needs none). */
+/* Bytes of scratch to give it_attn_f16 for this call geometry: more changes nothing (0: none is used).
+ * Less is accepted too, see it_attn_f16. A prompt call (nt >= 16) may use only part of them, or none where
+ * one pass is faster, and they do not grow evenly with pos0 (the ranges of keys change): one buffer for many
+ * calls takes the largest over their geometries, or it_attention_dispatch_room, which is always enough. */
 size_t it_attn_scratch_bytes(int pos0, int nt, int hd, int nh, int nkv);
 
 /* Causal GQA attention with sigmoid output gate, f32 accumulation.
@@ -86,9 +89,9 @@ size_t it_attn_scratch_bytes(int pos0, int nt, int hd, int nh, int nkv);
  *   out  : f32 out[t*out_tok_stride + h*hd + d] = softmax(scale*q.K) V * sigmoid(gate).
  *   scratch: device buffer for the partial records (split-K: 260 f32 words per token, head and split;
  *          flash key splits: 132 words, O as int16). it_attn_scratch_bytes(...) bytes give the
- *          library's preferred split; with fewer bytes the keys per split double until the records
- *          fit (the reference's rule for its fixed arena, src/vk/mod.rs:714-716), and the prefill
- *          kernel falls back to one pass with no scratch. The reference's own room,
+ *          library's preferred split; with fewer, decode and verify calls double the keys per split
+ *          until the records fit (the reference's rule for its fixed arena, src/vk/mod.rs:714-716) and
+ *          prompt calls take the fastest split whose records fit, or one pass with no scratch. The reference's own room,
  *          it_attention_dispatch_room(ctx_len, nh, nt) * 4 bytes, is always enough. NULL = 0 bytes.
  * Requires hd == 256, nh % nkv == 0, q_tok_stride and out_tok_stride multiples of 4, 16-byte
  * aligned q/out/kc/vc (the reference asserts the same f16 layout, src/vk/mod.rs:713).
@@ -181,13 +184,14 @@ int it_attn_f16_mailbox(const float* q, int q_tok_stride, const uint16_t* kc, co
                         void* mailbox, size_t mailbox_bytes, void* scratch, size_t scratch_bytes, void* stream);
 
 /* The choice it_attn_f16 makes for this geometry and scratch budget: *kernel 1 (split-K) or 2
- * (flash), *chunk keys per split (0 = flash in one pass), *bytes of scratch it takes room for (flash
- * may use less of it: longer splits, or one pass, where they are faster).
+ * (flash), *chunk keys per split (0 = flash in one pass), *bytes of scratch to give the call:
+ * it_attn_scratch_bytes where the budget holds them (flash may use less, or none), else what the
+ * records of the split take. A call with *bytes of scratch makes the same choice.
  * Returns nonzero if no split fits (only possible for nt < 16 with fewer than nt*nh*1040 bytes).
  * Scratch per split: the split-K kernel's records are 260 f32 words per (token, head); the flash
  * kernel's key-split records are 132 words per (token, head): {m, l, k, 0} and O as int16 in
  * units of k = max|O| / 32767 (an error of at most max|O| / 65534 per value before the merge).
- * Host-only; the chunk loop is the reference's, src/vk/mod.rs:714-716. */
+ * Host-only; the split-K chunk loop is the reference's, src/vk/mod.rs:714-716. */
 int it_attn_plan(int pos0, int nt, int hd, int nh, int nkv, size_t scratch_bytes, int* kernel, int* chunk,
                  size_t* bytes);
 

@@ -78,28 +78,34 @@ size_t flash_scratch(int pos0, int nt, int nh, int chunk, bool f32rec = false) {
     return (size_t)nt * nh * smax * (f32rec ? PART_WORDS : (size_t)it::FLASH_REC) * sizeof(float);
 }
 
-// Kernel and keys per split for an automatic call that must fit `budget` bytes of scratch. The
-// library's preferred split is kept when it fits; otherwise the split doubles until the records
-// fit, which is the reference's rule for its fixed arena (src/vk/mod.rs:714-716: C doubles from 64
-// while nt*nh*ceil((pos0+nt)/C)*260 words exceed the room). The flash kernel ends at one pass over
-// all keys, which needs no scratch, so it always has a plan; the split-K kernel (nt < 16) can run
-// out of doublings only when even one record per (token, head) exceeds the budget. A chunk of 0
-// from the flash plan means the one-pass form. Returns false if nothing fits. `bytes` is the room of the
-// split so found; the flash kernel may run longer ranges in it, or one pass, where that is faster
-// (flash_run_chunk), and `chunk` is what it runs.
-struct AttnPlan { int kernel, chunk; size_t bytes; };
+// Kernel and keys per split for an automatic call that must fit `budget` bytes of scratch.
+// Split-K (nt < 16): the library's preferred split is kept when it fits; otherwise the split doubles
+// until the records fit, which is the reference's rule for its fixed arena (src/vk/mod.rs:714-716: C
+// doubles from 64 while nt*nh*ceil((pos0+nt)/C)*260 words exceed the room). It can run out of
+// doublings only when even one record per (token, head) exceeds the budget: returns false.
+// Flash: of the ranges whose records fit the budget, and the room the library asks for
+// (flash_split_chunk), those that are fastest (flash_run_chunk); more scratch than asked for changes
+// nothing. A chunk of 0 means one pass over all keys, which needs no scratch, so there is always a
+// plan. `bytes` is the room asked for where the budget holds it (the launch may use less of it, or
+// none), else what the records of the split take. `split_room`: the budget holds the records of a
+// split of this call, so its scratch is held to the records' alignment, whichever form is faster.
+struct AttnPlan { int kernel, chunk; size_t bytes; bool split_room; };
 bool plan_attn(int pos0, int nt, int nh, int nkv, int kernel, size_t budget, AttnPlan& p) {
     const long total = (long)pos0 + nt;
     if (kernel == KERNEL_AUTO) kernel = auto_kernel(nt);
     p.kernel = kernel;
     if (kernel == KERNEL_FLASH || kernel == KERNEL_FLASH_F32) {
         const bool f32 = kernel == KERNEL_FLASH_F32;
-        int c = flash_chunk(pos0, nt, nh, nkv, 0);
-        while (c && flash_scratch(pos0, nt, nh, c, f32) > budget) c = (2L * c >= total) ? 0 : 2 * c;
-        p.chunk = c ? it::flash_run_chunk(pos0, nt, nh, nkv, c) : 0;
-        p.bytes = c ? flash_scratch(pos0, nt, nh, c, f32) : 0;
+        const int pref = flash_chunk(pos0, nt, nh, nkv, 0);
+        const size_t room = pref ? flash_scratch(pos0, nt, nh, pref, f32) : 0;
+        const size_t one = flash_scratch(pos0, nt, nh, (int)total, f32);   // the records of one range
+        const size_t ranges = (budget < room ? budget : room) / one;
+        p.split_room = ranges >= 2;
+        p.chunk = p.split_room ? it::flash_run_chunk(pos0, nt, nh, nkv, (int)ranges) : 0;
+        p.bytes = room <= budget ? room : p.chunk ? flash_scratch(pos0, nt, nh, p.chunk, f32) : 0;
         return true;
     }
+    p.split_room = true;
     int c = auto_chunk(pos0, nt, nh, nkv);
     while (splitk_scratch(pos0, nt, nh, c) > budget && c < total) c *= 2;
     p.chunk = c;
@@ -402,8 +408,7 @@ static int attn_f16_impl(const float* q, int qts, const uint16_t* q16, int q16ts
         if (!plan_attn(pos0, nt, nh, nkv, kernel, scratch ? scratch_bytes : 0, p))
             return fail("it_attn_f16: scratch of %zu bytes cannot hold even one partial record per (token, head) "
                         "(%zu bytes)", scratch_bytes, p.bytes);
-        // (also where the launch then needs less of the room, or none)
-        if (p.bytes && !aligned16(scratch)) return fail("it_attn_f16: scratch must be 16-byte aligned");
+        if (p.split_room && !aligned16(scratch)) return fail("it_attn_f16: scratch must be 16-byte aligned");
         kernel = p.kernel;
         if ((kernel == KERNEL_FLASH || kernel == KERNEL_FLASH_F32) && p.chunk == 0) chunk = 1 << 30;   // one pass
         else chunk = p.chunk;

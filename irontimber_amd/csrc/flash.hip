@@ -876,20 +876,6 @@ static long flash_split_wgs(int pos0, int nt, int G, int nkv, int bm, int chunk)
     return n * nkv;
 }
 
-// Ranges to weigh: `keys` in smax .. 2 equal ones, or up to two tiles longer ones, of at least `least` keys. A
-// short last range is seen by fewer row tiles, which can save a round (700 tokens at 1500: three ranges of 768
-// keys make 260 workgroups, of 832 244).
-template <class F>
-static void flash_ranges(int keys, int least, int smax, F&& weigh) {
-    for (int s = smax, last = 0; s >= 2; --s) {
-        const int c0 = max(((keys + s - 1) / s + BN - 1) / BN * BN, least);
-        for (int c = max(c0, last + BN); c <= c0 + 2 * BN && c < keys; c += BN) {
-            last = c;
-            weigh(c);
-        }
-    }
-}
-
 // A key-split launch in 64-row workgroups (NW = 4)? Up to one per CU of them: at one chunk always faster than
 // half as many of 128 rows (16 tokens at 1000 13.7 -> 11.7 us, 64 at 4096 21.3 -> 19.3, 128 at 8000 35.2
 // -> 34.9); two to a CU they only equal 128 rows.
@@ -898,61 +884,56 @@ static bool flash_split_w4(int pos0, int nt, int G, int nkv, int chunk) {
 }
 
 // Keys per split that the records of a prompt call are given room for, when one pass would leave it short of
-// workgroups (fewer than 128 of 128 rows); 0 for one pass. A launch takes whole rounds of 256 workgroups of 128
-// rows, each as long as its longest split: the split minimises
-//   rounds * (1.8 us a 64-key tile + 12 us a workgroup) + 1 us per 32 workgroups of records to merge
-// over the splits into 1 .. 32 ranges (what the row merge holds: 24 tokens at 8000 in 63 ranges 24.4, in 32
-// 21.2 us), counting the workgroups that have keys to see. The launch itself may take longer ranges
-// (flash_run_chunk).
-// The split that reaches 256 workgroups without regard to the rounds left a second round of a few workgroups
-// at most sizes: 441 tokens at position 7560 (280 workgroups) 107 against 80 us, 24/4 heads with 64
-// tokens at 4096 34 against 26 us, 256 at 5000 75 against 49 us, 512 at 5000 132 against 99 us; where it had
-// met a whole round (16/2 heads, 64 and 512 tokens) the choice is the same.
+// workgroups (fewer than 128 of 128 rows): the split that reaches 256 of them, in at most 32 ranges (what the row
+// merge holds: 24 tokens at 8000 in 63 ranges 24.4, in 32 21.2 us). 0 for one pass. This bounds the records
+// (callers size their scratch by their bytes); the ranges that a launch takes in it are flash_run_chunk's.
 int flash_split_chunk(int pos0, int nt, int nh, int nkv) {
-    const int G = nh / nkv, R = nt * G, wgs = (R + BM - 1) / BM * nkv;
+    const int R = nt * (nh / nkv);
+    const int wgs = (R + BM - 1) / BM * nkv;
     const int keys = pos0 + nt;
     if (wgs >= 128 || keys <= 4 * BN) return 0;
-    const int smax = wgs <= 64 ? 32 : (2 * 256 + wgs - 1) / wgs;   // (beyond: always more rounds)
-    long best_cost = (long)(wgs + 255) / 256 * (288L * ((keys + BN - 1) / BN) + 1920);   // one pass; 1/160 us
-    int best = 0;
-    flash_ranges(keys, BN, smax, [&](int c) {
-        const long n = flash_split_wgs(pos0, nt, G, nkv, BM, c);
-        const long cost = (n + 255) / 256 * (288L * (c / BN) + 1920) + 5 * n;
-        if (cost <= best_cost) {
-            best_cost = cost;
-            best = c;
-        }
-    });
-    return best;
+    const int want = min((256 + wgs - 1) / wgs, 32);              // splits to reach ~256 workgroups
+    return ((keys + want - 1) / want + BN - 1) / BN * BN;         // whole 64-key tiles
 }
 
-// Keys per split that a launch with room for splits of `chunk` keys takes: ranges as long or longer, or 0 for
-// one pass, whichever is fastest by
+// Keys per split that a launch with room for the records of `splits` ranges takes, or 0 for one pass, whichever
+// is fastest by
 //   up to 256 workgroups of 64 rows   1.4 us a 64-key tile + 8.5 us
 //   else workgroups of 128 rows       rounds of 256 * (1.9 us a tile + 9 us)
 //                                     both + 1 us per 4096 record rows and 1 us per 2048 output rows to merge
 //   one pass, 64 rows                 1.4 us a tile + 8.5 us
-// Over 773 splits of 16 .. 1000 tokens at 0 .. 7200, 16/2 and 24/4 heads, the choice by these costs is on
-// average 0.2 % slower than the fastest measured one. At the room's own split and at the choice: 64 tokens at
-// 4096 (22 ranges, 13) 19.4 and 17.6 us, at 1000 14.6 and 12.2, 16 at 8000 19.3 and 16.0, 24/4 heads 64 at 4096
-// 26 and 21.5, 300 at 0 (one pass) 17.4 and 14.5, 1000 at 0 (one pass) 36.6 and 30.5.
-int flash_run_chunk(int pos0, int nt, int nh, int nkv, int chunk) {
+// Weighed are the keys in `splits` .. 2 equal ranges, or up to four tiles longer ones: a short last range is seen
+// by fewer row tiles, which can save a round (700 tokens at 1500: three ranges of 768 keys make 260 workgroups, of
+// 832 244).
+// Over 321 calls of 16 .. 1015 tokens at 0 .. 7232 with 16/2, 24/4, 8/1 and 32/2 heads, each also timed with 17
+// other splits and in one pass, the choice takes 0.3 % longer than the fastest with room (geometric mean; at worst 7 %:
+// 512 tokens at 704, 24/4 heads) and 0.7 % longer than the fastest of all; the split that gives the room 11 % longer:
+// 64 tokens at 4096 20.8 against 19.1 us, 16 at 1000 12.3 and 11.4, 24/4 heads 300 at 4096 73 and 51, 600 at 1000 57
+// and 45 (one pass). Ranges that would need more room are up to 11 % faster for 460 .. 760 tokens far on, in two rounds
+// (700 at 7168: six ranges, 35 MB of records, 120 us; two, in room for three, 133).
+int flash_run_chunk(int pos0, int nt, int nh, int nkv, int splits) {
     const int G = nh / nkv, keys = pos0 + nt;
+    const long merge = 5L * nt * nh / 64;
     long best_cost = 224L * ((keys + BN - 1) / BN) + 1360;   // 1/160 us
-    int best = 0;
-    flash_ranges(keys, chunk, (keys + chunk - 1) / chunk, [&](int c) {
-        const long n4 = flash_split_wgs(pos0, nt, G, nkv, 4 * RW, c);
-        long cost = 224L * (c / BN) + 1360 + 5 * n4 / 2;
-        if (n4 > 256) {
-            const long n8 = flash_split_wgs(pos0, nt, G, nkv, 8 * RW, c);
-            cost = (n8 + 255) / 256 * (304L * (c / BN) + 1440) + 5 * n8;
+    int best = 0, last = 0;                                  // (ranges are weighed in rising order)
+    for (int s = splits; s >= 2; --s) {
+        const int c0 = ((keys + s - 1) / s + BN - 1) / BN * BN;
+        for (int c = max(c0, last + BN); c <= c0 + 4 * BN && c < keys; c += BN) {
+            last = c;
+            long cost = 224L * (c / BN) + 1360 + merge;
+            if (cost >= best_cost) return best;              // (and so is every longer range's)
+            const long n4 = flash_split_wgs(pos0, nt, G, nkv, 4 * RW, c);
+            cost += 5 * n4 / 2;
+            if (n4 > 256) {
+                const long n8 = flash_split_wgs(pos0, nt, G, nkv, 8 * RW, c);
+                cost = (n8 + 255) / 256 * (304L * (c / BN) + 1440) + 5 * n8 + merge;
+            }
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = c;
+            }
         }
-        cost += 5L * nt * nh / 64;
-        if (cost < best_cost) {
-            best_cost = cost;
-            best = c;
-        }
-    });
+    }
     return best;
 }
 

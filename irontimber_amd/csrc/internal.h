@@ -57,7 +57,7 @@ hipError_t launch_attn_flash(const float* q, int qts, const uint16_t* kc, const 
                              const uint16_t* q16 = nullptr, int q16ts = 0);
 
 int flash_split_chunk(int pos0, int nt, int nh, int nkv);
-int flash_run_chunk(int pos0, int nt, int nh, int nkv, int chunk);
+int flash_run_chunk(int pos0, int nt, int nh, int nkv, int splits);
 hipError_t launch_attn_flash_split(const float* q, int qts, const uint16_t* kc, const uint16_t* vc, int kvd, int pos0,
                                    int nh, int nkv, int nt, float scale, float* out, int ots, float* part, int chunk,
                                    hipStream_t st, bool f32rec = false, const uint16_t* q16 = nullptr,

@@ -235,6 +235,41 @@ def test_misaligned_scratch_refused_where_room_is_planned():
         assert "aligned" in _lib.last_error()
 
 
+@pytest.mark.parametrize("nh,nkv", [(16, 2), (24, 4), (8, 1)])
+def test_flash_room_is_bounded(nh, nkv):
+    """Records asked for by prompt calls: below 128 workgroups of 128 rows, splits reach 256 of them, so never
+    more than 255 + 127 tiles' records (128 rows of 528 bytes)."""
+    for nt in range(16, 1200, 23):
+        for pos0 in range(0, 8193 - nt, 61):
+            assert _lib.lib().it_attn_scratch_bytes(pos0, nt, 256, nh, nkv) <= 382 * 128 * 528, (pos0, nt)
+
+
+@pytest.mark.parametrize("nh,nkv", [(16, 2), (24, 4), (8, 1)])
+def test_flash_plan_takes_a_split_that_fits(nh, nkv):
+    """Prompt calls with less room than asked for: the plan fits, the same call with the planned bytes makes
+    the same choice, and room for the preferred split's own records (or more than asked for) keeps that split."""
+    for nt in (16, 17, 64, 100, 300, 441, 676, 1000):
+        for pos0 in range(0, 8193 - nt, 123):
+            one = nt * nh * 528
+            rc, kernel, pref, room = plan(pos0, nt, nh, nkv, 1 << 40)
+            assert (rc, kernel) == (0, 2) and room % one == 0 and plan(pos0, nt, nh, nkv, room) == (0, 2, pref, room)
+            if pref:
+                own = -(-(pos0 + nt) // pref) * one
+                assert own <= room and plan(pos0, nt, nh, nkv, own)[2] == pref, (pos0, nt)
+            for ranges in range(0, room // one):
+                rc, _, chunk, used = plan(pos0, nt, nh, nkv, ranges * one + one // 2)
+                assert rc == 0 and used == (-(-(pos0 + nt) // chunk) * one if chunk else 0) and used <= ranges * one
+                assert used == 0 or plan(pos0, nt, nh, nkv, used)[2] == chunk, (pos0, nt, ranges)
+
+
+def test_flash_split_in_little_room():
+    """Room that an unused shorter split does not divide evenly still holds the ranges that fit it: 64 tokens at 4096
+    in 13 ranges of 320 keys, 676 at 1246 in three of 704 rather than one pass."""
+    assert plan(4096, 64, 16, 2, 13 * 64 * 16 * 528) == (0, 2, 320, 13 * 64 * 16 * 528)
+    rc, _, chunk, used = plan(1246, 676, 16, 2, 3 * 676 * 16 * 528)
+    assert rc == 0 and 0 < chunk <= 704 and used <= 3 * 676 * 16 * 528
+
+
 def plan(pos0, nt, nh, nkv, budget):
     k, c, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
     rc = _lib.lib().it_attn_plan(pos0, nt, 256, nh, nkv, budget, ctypes.byref(k), ctypes.byref(c), ctypes.byref(b))
