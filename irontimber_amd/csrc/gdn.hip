@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void gdn_conv_l2_kernel(const float* __restric
     }
 }
 
-// The same pass with 16-byte accesses (strides and bases 16-byte aligned, cd % 256 == 0): lane l
+// The same pass with 16-byte accesses (strides and bases but the taps' 16-byte aligned, cd % 256 == 0): lane l
 // holds channels 256*wb + 4l .. 4l+3 of wave block wb, so lanes 0-31 and 32-63 each hold one
 // 128-channel head and a head's sum of squares is a reduction over its 32 lanes (DPP within the
 // 16-lane rows, then a row swap). A quarter of the memory instructions of the scalar form. For prompts
@@ -170,10 +170,12 @@ __global__ __launch_bounds__(256) void gdn_conv_l2_v4_kernel(const float* __rest
     f4 xs[TMAX], wt[K], win[K - 1];
 #pragma unroll
     for (int j = 0; j < TMAX; ++j) xs[j] = ld_f4(x + (size_t)(t0 + min(j, n - 1)) * xts + ch);
-    // taps of channel ch + e: floats (ch + e) * K .. + K, the lane's 4K floats as K aligned f4
+    // taps of channel ch + e: floats (ch + e) * K .. + K, the lane's 4K floats as K f4 (the taps may
+    // start at any float)
+    typedef float f4w __attribute__((ext_vector_type(4), aligned(4)));
     f4 wv[K];
 #pragma unroll
-    for (int i = 0; i < K; ++i) wv[i] = ld_f4(w + (size_t)ch * K + 4 * i);
+    for (int i = 0; i < K; ++i) wv[i] = *(const f4w*)(w + (size_t)ch * K + 4 * i);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -710,11 +712,12 @@ hipError_t launch_gdn_conv_l2(const float* x, int xts, const float* w, float* st
                               bool defer_state) {
     const int TT = nt <= 16 ? nt : 16;
     const dim3 grid((cd / 128 + 3) / 4, (nt + TT - 1) / TT);
-    // 16-byte form for prompts (several 16-token runs) when every access is 16-byte aligned and a
+    // 16-byte form for prompts (several 16-token runs) when the rows are 16-byte aligned and a
     // wave's 256 channels are whole; a decode or verify token keeps twice the waves of the scalar form
     // (a grid has at most 65535 rows of runs: longer prompts take the scalar form's 16-token runs)
-    const bool v4 = nt > 16 && nt <= 8 * 65535 && cd % 256 == 0 && xts % 4 == 0 && ots % 4 == 0 && ((uintptr_t)x & 15) == 0 &&
-                    ((uintptr_t)out & 15) == 0 && ((uintptr_t)state & 15) == 0 && ((uintptr_t)w & 15) == 0 && (!ck || ((uintptr_t)ck & 15) == 0);
+    const bool v4 = nt > 16 && nt <= 8 * 65535 && cd % 256 == 0 && xts % 4 == 0 && ots % 4 == 0 &&
+                    ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)state & 15) == 0 &&
+                    (!ck || ((uintptr_t)ck & 15) == 0);
     // Tokens a run: 4 for prompts of up to 2^23 values (x + its f16 or f32 output stay near the L2s and the
     // pass is bound by one round trip per wave with too few waves in flight), 8 beyond (each run reads
     // the K-1 rows before it again, which then come from memory). Prefill layer, 16 / 8 / 4 tokens a run:

@@ -474,7 +474,7 @@ def test_prefill_one_call_config5(dev):
 def test_conv_runs_and_prefill_conv_state(dev, nt, nv, nk, K):
     """The prompt conv at the edges of its 4-token runs, and of its 8-token runs (above 2^23 values):
     against the oracle; and the conv state that the one-call prefill leaves is the layer input's
-    last K-1 rows. Taps off by a float take the scalar form: the same to rounding."""
+    last K-1 rows. Taps off by a float: the same to rounding."""
     announce(f"conv runs nt={nt} nv={nv} K={K}")
     d = gdn_inputs(51 + nt, nt=nt, nv=nv, nk=nk)
     w, st0 = d["w"][:, :K].copy(), d["conv_state"][:K - 1].copy()
@@ -493,6 +493,21 @@ def test_conv_runs_and_prefill_conv_state(dev, nt, nv, nk, K):
     ops.gdn_prefill(x, wd, st, dev_f32(d["beta_raw"], dev), dev_f32(d["alpha_raw"], dev), dev_f32(d["dt"], dev),
                     dev_f32(d["a"], dev), dev_f32(d["state"], dev), nv, nk)
     np.testing.assert_array_equal(host(st), wst)
+
+
+@pytest.mark.parametrize("nt,nv,nk,K", [(17, 8, 4, 4), (24, 8, 4, 3), (67, 32, 16, 2), (1029, 32, 16, 4)])
+def test_conv_taps_at_any_float(dev, nt, nv, nk, K):
+    """Taps one to three floats off a 16-byte boundary run the prompt conv in the same form: the same bits."""
+    announce(f"conv taps nt={nt} nv={nv} K={K}")
+    d = gdn_inputs(91 + nt, nt=nt, nv=nv, nk=nk)
+    x, w = dev_f32(d["x"], dev), dev_f32(d["w"][:, :K].copy(), dev)
+    runs = []
+    for off in range(4):
+        wd = torch.empty(w.numel() + off, device=dev)[off:].view(w.shape)
+        wd.copy_(w)
+        runs.append(host(ops.gdn_conv_l2norm(x, wd, dev_f32(d["conv_state"][:K - 1].copy(), dev), 2 * nk)))
+    for got in runs[1:]:
+        np.testing.assert_array_equal(got, runs[0])
 
 
 @pytest.mark.parametrize("nt,nv,nk", [(64, 40, 8), (65, 48, 16), (128, 64, 16), (193, 72, 24), (257, 33, 11)])
