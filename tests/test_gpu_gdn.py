@@ -510,6 +510,26 @@ def test_conv_taps_at_any_float(dev, nt, nv, nk, K):
         np.testing.assert_array_equal(got, runs[0])
 
 
+@pytest.mark.parametrize("nt,K,ck_after", [(17, 4, 0), (40, 4, 1), (40, 3, 16), (1029, 4, 1028)])
+def test_conv_checkpoint_at_any_float(dev, nt, K, ck_after):
+    """A prompt conv with a checkpoint gives the same bits wherever the checkpoint buffer starts, and the
+    checkpoint is the last K-1 inputs up to that token."""
+    announce(f"conv ckpt nt={nt} K={K} after={ck_after}")
+    nv, nk = (32, 16) if nt > 1000 else (8, 4)
+    d = gdn_inputs(95 + nt, nt=nt, nv=nv, nk=nk)
+    st0 = d["conv_state"][:K - 1].copy()
+    x, w = dev_f32(d["x"], dev), dev_f32(d["w"][:, :K].copy(), dev)
+    want = np.concatenate([st0, d["x"]])[ck_after + 1:ck_after + K]
+    runs = []
+    for off in range(2):
+        ck = torch.empty(st0.size + off, device=dev)[off:].view(st0.shape)
+        st = dev_f32(st0, dev)
+        runs.append(host(ops.gdn_conv_l2norm(x, w, st, 2 * nk, ckpt=ck, ckpt_after=ck_after)))
+        np.testing.assert_array_equal(host(ck), want)
+        np.testing.assert_array_equal(host(st), d["x"][nt - (K - 1):])
+    np.testing.assert_array_equal(runs[1], runs[0])
+
+
 @pytest.mark.parametrize("nt,nv,nk", [(64, 40, 8), (65, 48, 16), (128, 64, 16), (193, 72, 24), (257, 33, 11)])
 def test_scan_column_blocks(dev, nt, nv, nk):
     """Head counts whose scan takes 32 state columns a workgroup (more than 32 V heads), with one to five
