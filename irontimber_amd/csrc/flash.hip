@@ -457,6 +457,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_flash_w_kernel(
     const uint16_t* __restrict__ vc, int kvd, int pos0, int nh, int nkv, int nt, float scale, float* __restrict__ out,
     int ots, float* __restrict__ part, int chunk, int smax) {
     static_assert(NW == 4 || (NW == 8 && QM != 2), "eight waves: key splits only");
+    static_assert(!(F32REC && QM != 0), "f32 records: q as f32");
     constexpr bool DB = NW == 8;     // double-buffered tiles
     const bool by_keys = NW == 8 || part != nullptr;   // key splits and records, or one pass
     constexpr int BM = RW * NW;      // query rows per workgroup
@@ -956,13 +957,10 @@ hipError_t launch_attn_flash_split(const float* q, int qts, const uint16_t* kc, 
                                                                     scale, out, ots, part, chunk, smax)
 #define IT_FLASH_SPLIT_N(F32_, Q16_)                                                                                   \
     (nw == 4 ? IT_FLASH_SPLIT(4, F32_, Q16_) : IT_FLASH_SPLIT(8, F32_, Q16_))
-    if (f32rec) {
-        if (q16) IT_FLASH_SPLIT_N(true, 1);
-        else IT_FLASH_SPLIT_N(true, 0);
-    } else {
-        if (q16) IT_FLASH_SPLIT_N(false, 1);
-        else IT_FLASH_SPLIT_N(false, 0);
-    }
+    // (no entry point asks for f32 records of a pre-converted q; q holds the same query)
+    if (f32rec) IT_FLASH_SPLIT_N(true, 0);
+    else if (q16) IT_FLASH_SPLIT_N(false, 1);
+    else IT_FLASH_SPLIT_N(false, 0);
 #undef IT_FLASH_SPLIT_N
 #undef IT_FLASH_SPLIT
     hipError_t e = hipGetLastError();
