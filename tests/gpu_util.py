@@ -1,8 +1,11 @@
 """Helpers for the GPU parity tests: numpy <-> device tensors, named progress lines."""
+import ctypes
 import sys
 
 import numpy as np
 import torch
+
+from irontimber_amd._lib import lib
 
 
 def dev_f32(a, dev):
@@ -54,3 +57,22 @@ def assert_argmax_agrees(got: np.ndarray, want: np.ndarray, n_cls: int = 997, se
     assert bad.size == 0, f"argmax differs on {bad.size} rows with margins above {sigmas} sigma: {bad[:8]}"
     print(f"argmax: {rows.size} near-tie rows of {g.shape[0]} (margins {margin.max():.2e} <= {sigmas} sigma)")
     return int(rows.size)
+
+
+def flash_split_form(pos0, nt, nh, nkv):
+    """What an automatic prompt call launches when it has all the scratch it asks for: (keys per range, waves a
+    workgroup, whether only the workgroups with keys are launched); (0, 0, False) for one pass. A range has 64-row
+    workgroups (four waves) while at most 256 of them see keys, and the launch drops those without keys when there
+    would be more than 256 in all."""
+    k, c, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    assert lib().it_attn_plan(pos0, nt, 256, nh, nkv, 1 << 40, ctypes.byref(k), ctypes.byref(c), ctypes.byref(b)) == 0
+    chunk, rows = c.value, nt * (nh // nkv)
+    if k.value != 2 or not chunk:
+        return 0, 0, False
+    splits = -(-(pos0 + nt) // chunk)
+
+    def tiles(bm):   # (row tiles x ranges x KV heads, those with keys to see)
+        ends = [min(r + bm, rows) for r in range(0, rows, bm)]
+        return len(ends) * splits * nkv, nkv * sum(-(-(pos0 + -(-e // (nh // nkv))) // chunk) for e in ends)
+    waves = 4 if tiles(64)[1] <= 256 else 8
+    return chunk, waves, tiles(16 * waves)[0] > 256

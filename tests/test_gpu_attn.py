@@ -7,7 +7,7 @@ import oracle
 from oracle.ref_np import attn_f64, f16_to_f64
 from irontimber_amd import ops
 from irontimber_amd.synth import attn_inputs, f16_bits, f16_bits_rtz
-from tests.gpu_util import announce, assert_argmax_agrees, dev_f16bits, dev_f32, host
+from tests.gpu_util import announce, assert_argmax_agrees, dev_f16bits, dev_f32, flash_split_form, host
 from tests.r012 import CASES, GEOMS, arena
 
 pytestmark = pytest.mark.gpu
@@ -53,6 +53,29 @@ def test_attn_q16_bit_equal(dev, ctx, nt):
     np.testing.assert_array_equal(a, b)
     want = oracle.attn(q2, kb, vb, pos0, nh, nkv)
     assert np.abs(b - want).max() <= TOL
+
+
+@pytest.mark.parametrize("ctx,nt,nh,nkv,waves,packed", [
+    (8192, 512, 16, 2, 8, False), (8001, 441, 16, 2, 8, False), (7300, 300, 16, 2, 8, True),
+    (5256, 256, 24, 4, 8, False), (1512, 512, 24, 4, 8, True), (4160, 64, 24, 4, 4, False),
+    (1015, 295, 16, 2, 4, True), (1427, 187, 24, 4, 4, True)])
+def test_attn_q16_bit_equal_splits(dev, ctx, nt, nh, nkv, waves, packed):
+    """As above for the automatic key splits, in every form that their launch takes: workgroups of four and of eight
+    waves, all of them or only those with keys, both head geometries."""
+    pos0 = ctx - nt
+    chunk, *form = flash_split_form(pos0, nt, nh, nkv)
+    assert chunk and form == [waves, packed]
+    announce(f"attn q16 splits ctx={ctx} nt={nt} nh={nh}/{nkv} chunk={chunk}")
+    q, kb, vb = attn_inputs(63 + ctx, ctx=ctx, nt=nt, nh=nh, nkv=nkv)
+    qd, kc, vc = dev_f32(q.reshape(nt, -1), dev), dev_f16bits(kb, dev), dev_f16bits(vb, dev)
+    s = float(np.float32(np.float32(1.0 / 16) * np.float32(1.4426950408889634)))
+    qh = (qd.view(nt, nh, 512)[:, :, :256] * s).half().reshape(nt, -1).contiguous()
+    a, b = host(ops.attn_f16(qd, kc, vc, pos0, nh, nkv)), host(ops.attn_f16_q16(qd, qh, kc, vc, pos0, nh, nkv))
+    np.testing.assert_array_equal(a, b)
+    for t0 in sorted({0, nt // 2 - 8, nt - 16}):
+        want = oracle.attn(q[t0:t0 + 16].reshape(16, -1), kb, vb, pos0 + t0, nh, nkv)
+        assert np.isfinite(b).all() and np.abs(b[t0:t0 + 16] - want).max() <= TOL
+
 
 @pytest.mark.parametrize("ctx,nt,nh,nkv", [(1, 1, 16, 2), (65, 1, 16, 2), (100, 3, 16, 2), (64, 2, 24, 4),
                                            (300, 5, 8, 8), (129, 7, 4, 1), (777, 33, 16, 2), (64, 64, 16, 2)])
@@ -153,16 +176,20 @@ def test_flash_whole_prompt_8192(dev):
 
 
 @pytest.mark.parametrize("ctx,nt,nh,nkv", [(4160, 64, 24, 4), (8001, 441, 16, 2), (5256, 256, 24, 4),
-                                           (8024, 24, 16, 2), (317, 17, 16, 2), (700, 700, 16, 2), (3700, 700, 16, 2)])
+                                           (8024, 24, 16, 2), (317, 17, 16, 2), (272, 16, 16, 2), (3700, 700, 16, 2),
+                                           (1700, 700, 16, 2), (8008, 1008, 16, 2), (640, 128, 24, 4),
+                                           (588, 300, 24, 4), (1512, 512, 24, 4), (7860, 660, 24, 4)])
 def test_flash_split_plans(dev, ctx, nt, nh, nkv):
     """The automatic key splits of prompt calls over both head geometries, ragged lengths and the
     smallest and largest row counts that are split, against the oracle."""
+    assert flash_split_form(ctx - nt, nt, nh, nkv)[0] > 0
     got, want = run_case(dev, 61, ctx, nt, nh, nkv)
     assert np.isfinite(got).all() and np.abs(got - want).max() <= TOL
 
 
 @pytest.mark.parametrize("ctx,nt,nh,nkv", [(8, 8, 16, 2), (9, 9, 16, 2), (12, 11, 24, 4), (129, 65, 16, 2),
-                                           (1025, 1025, 16, 2), (1400, 1400, 24, 4), (2100, 2100, 16, 2),
+                                           (700, 700, 16, 2), (1025, 1025, 16, 2), (1400, 1400, 24, 4),
+                                           (2100, 2100, 16, 2),
                                            (3100, 3100, 16, 2), (2300, 1030, 16, 2), (2100, 2100, 24, 4)])
 def test_flash_64_row_one_pass(dev, ctx, nt, nh, nkv):
     """One pass in workgroups of 64 rows (16-row waves): a wave, a tile and one past it, two workgroups a CU in

@@ -12,7 +12,7 @@ import oracle
 from irontimber_amd import ops
 from irontimber_amd._lib import lib
 from irontimber_amd.synth import attn_inputs, gdn_inputs
-from tests.gpu_util import announce, dev_f16bits, dev_f32, host
+from tests.gpu_util import announce, dev_f16bits, dev_f32, flash_split_form, host
 
 pytestmark = pytest.mark.gpu
 GUARD = 1 << 16
@@ -53,6 +53,23 @@ def test_attention_scratch_bands(dev, ctx, nt, nh, nkv, kernel, chunk):
     assert_bands(buf, n)
     want = oracle.attn(q.reshape(nt, -1), kb, vb, pos0, nh, nkv)
     assert np.abs(got - want).max() <= 2e-3
+
+
+@pytest.mark.parametrize("ctx,nt,nh,nkv", [(8192, 512, 16, 2), (7300, 300, 16, 2), (1015, 295, 16, 2),
+                                           (4096 + 64, 64, 16, 2), (1512, 512, 24, 4)])
+def test_flash_split_bands(dev, ctx, nt, nh, nkv):
+    """Prompt calls given only the records of the ranges they take (the library asks for room for more)."""
+    pos0 = ctx - nt
+    chunk, waves, packed = flash_split_form(pos0, nt, nh, nkv)
+    n = ops.attn_scratch_bytes(pos0, nt, nh, nkv, 256, ops.KERNEL_FLASH, chunk)
+    announce(f"bands flash ctx={ctx} nt={nt} nh={nh}/{nkv} chunk={chunk} waves={waves} packed={packed} bytes={n}")
+    assert chunk and n > 0
+    q, kb, vb = attn_inputs(45, ctx=ctx, nt=nt, nh=nh, nkv=nkv)
+    qd, kc, vc = dev_f32(q.reshape(nt, -1), dev), dev_f16bits(kb, dev), dev_f16bits(vb, dev)
+    buf, scr = banded(n, dev)
+    got = host(ops.attn_f16(qd, kc, vc, pos0, nh, nkv, scratch=scr))
+    assert_bands(buf, n)
+    np.testing.assert_array_equal(got, host(ops.attn_f16(qd, kc, vc, pos0, nh, nkv)))   # the same ranges
 
 
 @pytest.mark.parametrize("rows,nt,nh,nkv,splits", [(8192, 1, 16, 2, 0), (8192, 2, 16, 2, 0), (4096 + 64, 64, 16, 2, 0),
