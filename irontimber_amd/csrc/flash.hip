@@ -107,9 +107,14 @@ __global__ __launch_bounds__(256) void attn_flash_kernel(
     // head, the last one's heavy row tiles start when most of the launch is done (24/4 heads: 2048 tokens 98
     // -> 76 us, 2500 125 -> 104, 4096 263 -> 254). With two heads or one, each heavy row tile is in the first
     // round of 256 either way and head after head is up to 2 % faster after a context and at 5000 - 6000
-    // tokens, up to 2 % slower at 3500 - 4096.
-    const int id = blockIdx.x;
-    const int rt = nrt - 1 - (nkv > 2 ? id / nkv : id % nrt), kh = nkv > 2 ? id % nkv : id / nrt;
+    // tokens, up to 2 % slower at 3500 - 4096. So it is with three or four just past two rounds, after a context of
+    // a third of the tokens or more: the few row tiles of the third round are then nearly as heavy as the others, and
+    // side by side they start when every CU has done its two (24/4 heads, side by side and head after head: 2933
+    // tokens, 552 workgroups, at 1759 298 and 279 us, at 2933 400 and 377; 3300, 620, at 1700 324 and 317; but 3413,
+    // 640, at 2400 397 and 404, 2666, 500, at 2666 287 and 312).
+    const int id = blockIdx.x, n = nrt * nkv;
+    const bool abreast = nkv > 2 && !(nkv <= 4 && n > 512 && n <= 624 && 3L * pos0 >= nt);
+    const int rt = nrt - 1 - (abreast ? id / nkv : id % nrt), kh = abreast ? id % nkv : id / nrt;
     // the wave index as a scalar: row counts, row walks and branches on them stay in SGPRs
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, hh = l >> 5, c = l & 31;
     const int r = rt * BM + 32 * w + c;                 // this lane's query row

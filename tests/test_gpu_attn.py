@@ -210,6 +210,23 @@ def test_flash_64_row_one_pass(dev, ctx, nt, nh, nkv):
             assert np.isfinite(got).all() and np.abs(got[t0:t0 + n] - want).max() <= TOL
 
 
+@pytest.mark.parametrize("pos0,nt,nh,nkv", [(1400, 2752, 24, 4), (1400, 2720, 24, 4), (900, 2752, 24, 4),
+                                            (1500, 2760, 24, 3), (1200, 3350, 24, 4)])
+def test_flash_row_tile_orders(dev, pos0, nt, nh, nkv):
+    """One pass in workgroups of 128 rows, three and four KV heads, on both sides of the rule that orders their row
+    tiles (512 and 624 workgroups, a context of a third of the tokens): every token's output is there, and those around the tile
+    edges and at both ends match the oracle."""
+    announce(f"flash order pos0={pos0} nt={nt} nh={nh}/{nkv}")
+    q, kb, vb = attn_inputs(69, ctx=pos0 + nt, nt=nt, nh=nh, nkv=nkv)
+    out = torch.full((nt, nh * 256), float("nan"), device=dev)
+    got = host(ops.attn_f16(dev_f32(q.reshape(nt, -1), dev), dev_f16bits(kb, dev), dev_f16bits(vb, dev), pos0, nh, nkv,
+                            out=out))
+    assert np.isfinite(got).all()
+    for t0 in (0, nt // 2, nt - 8):
+        want = oracle.attn(q[t0:t0 + 8].reshape(8, -1), kb, vb, pos0 + t0, nh, nkv)
+        assert np.abs(got[t0:t0 + 8] - want).max() <= TOL
+
+
 @pytest.mark.parametrize("nt,pos0,chunk", [(1, 700, 64), (9, 700, 128), (64, 4096, 320), (64, 4096, 256), (130, 500, 64)])
 @pytest.mark.parametrize("kernel", [ops.KERNEL_FLASH, ops.KERNEL_FLASH_F32])
 def test_flash_split_workgroup_rows(dev, nt, pos0, chunk, kernel):
