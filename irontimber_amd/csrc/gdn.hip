@@ -722,8 +722,16 @@ hipError_t launch_gdn_conv_l2(const float* x, int xts, const float* w, float* st
     // pass is bound by one round trip per wave with too few waves in flight), 8 beyond (each run reads
     // the K-1 rows before it again, which then come from memory). Prefill layer, 16 / 8 / 4 tokens a run:
     // 24 tokens x 8192 channels 19.3 / 16.9 / 15.9 us, 500 34.5 / 32.9 / 32.0, 1000 48.7 / 46.3 / 45.3;
-    // 500 x 10240 47.0 / 44.7 / 44.0, 1000 72.8 / 68.9 / 71.1, 4096 248 / 245 / 257 us.
-    const int TT4 = (size_t)nt * cd <= (1u << 23) ? 4 : 8;
+    // 500 x 10240 47.0 / 44.7 / 44.0, 1000 72.8 / 68.9 / 71.1, 4096 248 / 245 / 257 us. The f32 output leaves
+    // the L2s at half as many values, and where the pass then runs from the memory-side cache (to 34 M values)
+    // the rows read again cost most: 4 to 4.5 M, 16 at 16 - 34 M. The pass alone, 4 / 8 / 16: 1000 x 7168 15.2 / 14.5 /
+    // 15.0, 4096 x 2048 17.1 / 15.8 / 16.3, 4096 x 7168 48.8 / 43.9 / 41.7, 2800 x 10240 47.6 / 43.0 / 40.9, 4096 x
+    // 10240 68.8 / 62.5 / 64.4. Not for rows a multiple of 32 KB apart: 700 x 8192 11.2 / 12.2 / 14.1, 2800 x 8192
+    // 30.4 / 31.2 / 32.3.
+    const size_t values = (size_t)nt * cd, M = 1u << 20;
+    const bool spread = sizeof(OutT) == 4 && xts % 8192 != 0;
+    const bool mid = spread && values >= 16 * M && values <= 34 * M;
+    const int TT4 = 2 * values <= (spread ? 9 * M : 16 * M) ? 4 : mid ? 16 : 8;
     const dim3 grid4((cd / 256 + 3) / 4, (nt + TT4 - 1) / TT4);
 #define IT_L2_V4(KK, TM)                                                                                            \
     gdn_conv_l2_v4_kernel<KK, OutT, TM><<<grid4, 256, 0, st>>>(x, xts, w, state, out, ots, cd, nt, nnorm, eps)
@@ -734,7 +742,8 @@ hipError_t launch_gdn_conv_l2(const float* x, int xts, const float* w, float* st
     if (ck && grid.y > 1)                                                                                           \
         gdn_conv_state_kernel<KK><<<(cd + 255) / 256, 256, 0, st>>>(x, xts, state, ck, cd, ck_after + 1);          \
     if (v4 && TT4 == 4) IT_L2_V4(KK, 4);                                                                            \
-    else if (v4) IT_L2_V4(KK, 8);                                                                                   \
+    else if (v4 && TT4 == 8) IT_L2_V4(KK, 8);                                                                       \
+    else if (v4) IT_L2_V4(KK, sizeof(OutT) == 4 ? 16 : 8);   /* (f32 output only) */                                \
     else if (TT <= 1) IT_L2_RUN(KK, 1);                                                                             \
     else if (TT <= 2) IT_L2_RUN(KK, 2);                                                                             \
     else if (TT <= 4) IT_L2_RUN(KK, 4);                                                                             \

@@ -470,10 +470,10 @@ def test_prefill_one_call_config5(dev):
 
 
 @pytest.mark.parametrize("nt,nv,nk,K", [(17, 8, 4, 4), (18, 8, 4, 3), (19, 4, 2, 2), (24, 8, 4, 4), (67, 48, 16, 4),
-                                        (1029, 32, 16, 4)])
+                                        (1029, 32, 16, 4), (665, 40, 8, 2), (2405, 40, 8, 4), (2400, 40, 8, 3)])
 def test_conv_runs_and_prefill_conv_state(dev, nt, nv, nk, K):
-    """The prompt conv at the edges of its 4-token runs, and of its 8-token runs (above 2^23 values):
-    against the oracle; and the conv state that the one-call prefill leaves is the layer input's
+    """The prompt conv at the edges of its 4-token runs, of its 8-token runs (above 4.5 * 2^20 values, 2^23 at 8192
+    channels) and of its 16-token runs (above 2^24): against the oracle; and the conv state that the one-call prefill leaves is the layer input's
     last K-1 rows. Taps off by a float: the same to rounding."""
     announce(f"conv runs nt={nt} nv={nv} K={K}")
     d = gdn_inputs(51 + nt, nt=nt, nv=nv, nk=nk)
