@@ -123,7 +123,7 @@ bool plan_attn(int pos0, int nt, int nh, int nkv, int kernel, size_t budget, Att
 struct F32kvPlan { int chunk; size_t bytes; };
 // The f32-KV kernel's preferred split. Calls of one block of query rows (decode, verify: up to 32
 // rows per KV head) keep one 64-key tile per split. Calls with several row blocks (the 64-token
-// catch-up) read each K/V tile once per block and hold one workgroup per CU (133 KB of LDS), so
+// catch-up) read each K/V tile once per block and hold one workgroup per CU (142 KB of LDS), so
 // their time goes as the number of rounds of workgroups over the CUs times the tiles a workgroup
 // walks: the split (a multiple of 64 keys) minimises rounds x (tiles + 1), the + 1 standing for a
 // workgroup's fixed cost (q rows, first tile, records), ties going to the longer split (fewer

@@ -43,7 +43,7 @@ __device__ __forceinline__ f4 mfma16x16x4f32(float a, float b, f4 c) {
 // the record part[((t*nh + h)*smax + s)*260] = {m, l, 0, 0, o[256]} (m in natural-log units) goes out
 // straight from the accumulators, with no merge of the waves. RB = 2 (multi-token calls) makes each
 // K/V tile serve 32 rows: the 64-token catch-up reads the cache 16 times instead of 32. Its eight
-// waves put two on a SIMD (133 KB of LDS: one workgroup a CU), so one's LDS reads, exponentials and
+// waves put two on a SIMD (142 KB of LDS: one workgroup a CU), so one's LDS reads, exponentials and
 // barriers overlap the other's f32 matrix ops, which bound a tile (8,192 cycles a CU). With four
 // waves of both blocks each, 64 tokens at slot 1024 / 2048 / 4096 / 8128 took 31.9 / 43.6 / 68.5 / 110.7
 // us against 29.0 / 38.9 / 59.6 / 94.7, 14 tokens at 7800 41.4 against 37.2.

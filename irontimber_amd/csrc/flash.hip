@@ -402,7 +402,8 @@ __device__ __forceinline__ void tile_to_lds16(const uint16_t* __restrict__ src, 
     for (int i = 0; i < 32 / NW; ++i) {
         const int r = 64 / NW * w + 2 * i + (l >> 5);
         const unsigned off = (unsigned)min(r, rmax) * rowb + (unsigned)cj[i];
-        __builtin_amdgcn_global_load_lds((const void*)(base + off), (lds_void*)(lds + (64 / NW * w + 2 * i) * HD), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void*)(base + off), (lds_void*)(lds + (64 / NW * w + 2 * i) * HD), 16,
+                                         0, 0);
     }
 }
 
@@ -445,8 +446,8 @@ __device__ __forceinline__ void flash_job(int id, int nrt, int nkv, int& rt, int
 // each, one K and one V buffer: V of a tile loads under its scores, K of the next under its P.V, two
 // barriers a tile). NW = 4 streams K and V once per 64 rows, but its wave alone on a SIMD takes 1.4
 // us a tile where eight take 1.8, short launches reach twice as many CUs, and two workgroups of
-// different length share a CU: one pass over 64 tokens 10.6 -> 8.4, 1024 tokens 40.8 -> 32.0, 1531 55.6
-// -> 44.2 us; key splits of 64 tokens at 1000 16.2 -> 13.9, at 8128 26.4 -> 24.8 us (NW = 8 -> 4).
+// different length share a CU: one pass over 64 tokens 11.3 -> 8.9, 1000 tokens 40.6 -> 32.2, 1531 57.0
+// -> 45.0 us; key splits of 64 tokens at 1000 16.2 -> 13.9, at 8128 26.4 -> 24.8 us (NW = 8 -> 4).
 // F32REC: the key-split records in the split-K kernels' lossless f32 form instead ({m, l, 0, 0} +
 // O as 256 floats, 260 words, merged by the f32 combine), selectable through it_attn_f16_ex.
 // QM: where the q operand comes from. 0: the f32 q rows, scaled and converted here. 1 and 2: q16,
@@ -501,7 +502,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_flash_w_kernel(
     // byte offset of the logical chunk each lane's DMA slot holds, plus the KV head's column
     int cj[32 / NW];
 #pragma unroll
-    for (int i = 0; i < 32 / NW; ++i) cj[i] = 2 * (int)head_off + 16 * ((l & 31) ^ swz16(64 / NW * w + 2 * i + (l >> 5)));
+    for (int i = 0; i < 32 / NW; ++i)
+        cj[i] = 2 * (int)head_off + 16 * ((l & 31) ^ swz16(64 / NW * w + 2 * i + (l >> 5)));
     // q as the B operand of S^T = K Q^T: lane (c, g) holds dims 32ks + 8g .. +7 of query row c,
     // scaled into log2 units. QM 0 and 2 read the wave's 16 rows whole and transpose them through
     // 8 KB of the second K/V buffers, which the first tile does not use, or (single buffers) of V's, the

@@ -748,7 +748,8 @@ hipError_t launch_gdn_conv_l2(const float* x, int xts, const float* w, float* st
     else if (TT <= 2) IT_L2_RUN(KK, 2);                                                                             \
     else if (TT <= 4) IT_L2_RUN(KK, 4);                                                                             \
     else IT_L2_RUN(KK, 16);                                                                                         \
-    if (grid.y > 1 && !defer_state) gdn_conv_state_kernel<KK><<<(cd + 255) / 256, 256, 0, st>>>(x, xts, state, state, cd, nt);
+    if (grid.y > 1 && !defer_state)                                                                                 \
+        gdn_conv_state_kernel<KK><<<(cd + 255) / 256, 256, 0, st>>>(x, xts, state, state, cd, nt);
     switch (K) {
         case 2: IT_CONVL2(2) break;
         case 3: IT_CONVL2(3) break;

@@ -95,7 +95,8 @@ void gdn_chunk_prep(const CoT* __restrict__ co, int cts, const float* __restrict
     const int nch = (nt + C - 1) / C;
     if ((int)blockIdx.x >= nch * nv) {
         // the workgroups past the chunks write the conv state: the conv kernel, whose runs read the
-        // old one, is done. A launch of its own cost 4-5 us of a 58 us layer at 500 tokens.
+        // old one, is done. A launch of its own cost 2 us of a layer: 24 tokens x 8192 channels 17.3 -> 15.5 us,
+        // 500 x 10240 38.4 -> 36.6.
         const int ch = ((int)blockIdx.x - nch * nv) * PREP_THREADS + (int)threadIdx.x;
         if (ch < tail.cd)
             for (int i = 0; i < tail.K - 1; ++i)

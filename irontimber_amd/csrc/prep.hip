@@ -16,8 +16,9 @@ constexpr int PREP_WAVES = 4;
 
 // Rotation angle of frequency i at position p: theta = p * tsc^i, with tsc the caller's f32
 // theta_scale. The power (binary exponentiation over the 7 bits of i < 128, with no loop to leave
-// early: 0.14 us of a 2.67 us one-token launch) and the reduction to [-pi, pi] run in f64, so the f32 sin/cos see an argument accurate to f32 rounding even at
-// positions near 2^22 (the reference's f32 recurrences lose ~2e-4 rad by position 8191).
+// early: 0.14 us of a 2.67 us one-token launch) and the reduction to [-pi, pi] run in f64, so the
+// f32 sin/cos see an argument accurate to f32 rounding even at positions near 2^22 (the reference's
+// f32 recurrences lose ~2e-4 rad by position 8191).
 __device__ __forceinline__ void rope_angle(int p, int i, float tsc, float& c, float& s) {
     double pw = i & 1 ? (double)tsc : 1.0, b = (double)tsc;
 #pragma unroll
